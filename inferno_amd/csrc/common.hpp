@@ -44,7 +44,9 @@ struct PlanOut {
   uint4* l128;
   uint4* l64;
   uint4* l32;
-  uint32_t* counts;  // [3]: lengths of l128, l64, l32
+  uint4* l16;
+  uint32_t* counts;  // [4]: lengths of l128, l64, l32, l16
+  bool narrow;       // 16-row tiles only
 };
 
 constexpr int kWave = 64;        // CDNA wavefront width

@@ -149,17 +149,17 @@ __global__ void __launch_bounds__(256)
 constexpr int kMaxBlasDevices = 64;
 std::mutex g_blas_mu;
 hipblasLtHandle_t g_blas[kMaxBlasDevices] = {};
-std::map<std::tuple<int, int, int, int, int, int>, hipblasLtMatmulHeuristicResult_t> g_algo;
+std::map<std::tuple<int, int, int, int, int, int, int>, hipblasLtMatmulHeuristicResult_t> g_algo;
 
 int blas_error(const char* what, int status) {
   set_error(std::string("hipBLASLt ") + what + " failed (status " + std::to_string(status) + ")");
   return INFERNO_ERR_DEVICE;
 }
 
-// D[n][m] (row-major, fp32) = X[n][k] (row-major f16) . W[m][k]^T (row-major
+// D[n][m] (row-major, fp32) = X[n][k] (row-major f16, ldx apart) . W[m][k]^T (row-major
 // f16): column-major D^T = op(W)^T-view x X-view with op(A) = T.
-int blas_gemm(hipStream_t s, const uint16_t* W, const uint16_t* X, float* D, int m, int n, int k,
-              void* ws, hipDataType in_type = HIP_R_16F, float beta = 0.0f) {
+int blas_gemm(hipStream_t s, const uint16_t* W, const uint16_t* X, int ldx, float* D, int m, int n,
+              int k, void* ws, hipDataType in_type = HIP_R_16F, float beta = 0.0f) {
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxBlasDevices) {
     set_error("hipBLASLt: cannot query the current device");
@@ -189,12 +189,12 @@ int blas_gemm(hipStream_t s, const uint16_t* W, const uint16_t* X, float* D, int
     hipblasLtMatmulDescSetAttribute(op, HIPBLASLT_MATMUL_DESC_TRANSA, &tA, sizeof(tA));
     hipblasLtMatmulDescSetAttribute(op, HIPBLASLT_MATMUL_DESC_TRANSB, &tB, sizeof(tB));
     if ((st = hipblasLtMatrixLayoutCreate(&la, in_type, k, m, k)) != HIPBLAS_STATUS_SUCCESS ||
-        (st = hipblasLtMatrixLayoutCreate(&lb, in_type, k, n, k)) != HIPBLAS_STATUS_SUCCESS ||
+        (st = hipblasLtMatrixLayoutCreate(&lb, in_type, k, n, ldx)) != HIPBLAS_STATUS_SUCCESS ||
         (st = hipblasLtMatrixLayoutCreate(&lc, HIP_R_32F, m, n, m)) != HIPBLAS_STATUS_SUCCESS) {
       fail("matrix layout");
       break;
     }
-    const auto key = std::make_tuple(dev, m, n, k, int(in_type), beta != 0.0f ? 1 : 0);
+    const auto key = std::make_tuple(dev, m, n, k, ldx, int(in_type), beta != 0.0f ? 1 : 0);
     auto it = g_algo.find(key);
     if (it == g_algo.end()) {
       hipblasLtMatmulPreference_t pref = nullptr;
@@ -294,11 +294,11 @@ int launch_dense_blas(hipStream_t s, const void* gate, const void* up, const voi
                                                  256 * 256), T, H, Is);
   int st;
   if ((st = launch_expand(s, gate, up, down, H, Is, w.wgu, w.wd))) return st;
-  if ((st = blas_gemm(s, w.wgu, x16, w.gu, int(2 * Is), int(T), int(H), lib_ws))) return st;
+  if ((st = blas_gemm(s, w.wgu, x16, int(f16_pitch(H)), w.gu, int(2 * Is), int(T), int(H), lib_ws))) return st;
   const size_t n = T * Is;
   swiglu_f16_kernel<<<unsigned((n + 255) / 256), 256, 0, s>>>(w.gu, T, Is, w.h);
   INF_LAUNCHED();
-  return blas_gemm(s, w.wd, w.h, ys, int(H), int(T), int(Is), lib_ws);
+  return blas_gemm(s, w.wd, w.h, int(Is), ys, int(H), int(T), int(Is), lib_ws);
 }
 
 size_t blas_lib_workspace_bytes() { return kBlasWsBytes; }
@@ -344,7 +344,7 @@ int launch_router_blas(hipStream_t s, const uint16_t* x, const float* w, size_t 
   // the three terms [3][E][H] are one [3E][H] operand: one GEMM of 3E
   // columns fills the chip better than three of E (c5: 256 columns made
   // 256 tiles of 64 x 64, one workgroup per CU)
-  if (int st = blas_gemm(s, terms, x, d3, int(3 * E), int(T), int(H), lib_ws, HIP_R_16BF, 0.0f))
+  if (int st = blas_gemm(s, terms, x, int(H), d3, int(3 * E), int(T), int(H), lib_ws, HIP_R_16BF, 0.0f))
     return st;
   sum3_kernel<<<unsigned((T * E + 255) / 256), 256, 0, s>>>(d3, T, uint32_t(E), logits);
   INF_LAUNCHED();

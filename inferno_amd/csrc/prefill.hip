@@ -30,14 +30,19 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "gemv_common.hpp"
+#include "grouped_gemm.hpp"
 #include "routing_dev.hpp"
 
 namespace inferno {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+using grouped::GemmArgs;
+using grouped::as_h2;
+using grouped::as_u32;
+using grouped::dequant8;
+using grouped::half2v;
+using grouped::half8;
+using grouped::mix_mul;
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2a __attribute__((ext_vector_type(2), aligned(8)));
 
@@ -46,36 +51,7 @@ constexpr int kTileN = 128;      // weight rows per workgroup
 constexpr int kLdsPitch = 72;    // halfs per LDS token row (64 + 8 pad: conflict-free reads)
 constexpr size_t kGemmCUs = 256;  // MI355X CUs (fixed, so a shape takes the same kernel on any device)
 
-__device__ __forceinline__ half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
-__device__ __forceinline__ uint32_t as_u32(half2v v) { return __builtin_bit_cast(uint32_t, v); }
-
-// v(f) = f * mult + off for both f16 subnormal fields of a masked word, in f16.
-__device__ __forceinline__ uint32_t fma_pair(uint32_t fields, float mult, float off) {
-  const half2v f = as_h2(fields);
-  const half2v r = {(_Float16)__builtin_fmaf((float)f[0], mult, off),
-                    (_Float16)__builtin_fmaf((float)f[1], mult, off)};
-  return as_u32(r);
-}
-
-// Eight values from bytes 0..7 of (w0, w1) with the field under `mask` (the
-// same mask in both 16-bit halves, at bit position p): value = field * mult +
-// off, mult already holding the 2^(24 - p). Output order 0 2 1 3 4 6 5 7.
-__device__ __forceinline__ half8 dequant8(uint32_t w0, uint32_t w1, uint32_t mask, float mult,
-                                          float off) {
-  const uint32_t a = fma_pair(w0 & mask, mult, off);
-  const uint32_t b = fma_pair((w0 >> 8) & mask, mult, off);
-  const uint32_t c = fma_pair(w1 & mask, mult, off);
-  const uint32_t d = fma_pair((w1 >> 8) & mask, mult, off);
-  return __builtin_bit_cast(half8, make_uint4(a, b, c, d));
-}
-
 __device__ __forceinline__ uint32_t byte_of(uint32_t w, int i) { return (w >> (8 * i)) & 0xffu; }
-
-// f16 half `hi` of w, exactly widened, times m plus c in fp32 (v_fma_mix_f32).
-__device__ __forceinline__ float mix_mul(uint32_t w, int hi, float m, float c) {
-  const half2v h = as_h2(w);
-  return __builtin_fmaf((float)h[hi], m, c);
-}
 
 // ------------------------------------------------------------- A fragments
 // A lane (row i, k half kg) dequantises, for 64-value chunk QC of a K unit
@@ -275,22 +251,6 @@ struct Frag<INFERNO_Q8_0> {
 
 // ------------------------------------------------------------------ GEMM
 
-struct GemmArgs {
-  const uint8_t* w0;       // gate (or the down / single matrix)
-  const uint8_t* w1;       // up, null for one matrix
-  size_t stride;           // bytes per expert matrix
-  const uint16_t* xin;     // f16 input rows (k order 0 2 1 3 4 6 5 7), K halfs each
-  uint32_t in_div;         // input row = (sorted[c] or c) / in_div
-  const uint32_t* sorted;  // dispatch order, null = dense (identity)
-  const float* route_w;    // routing weight per assignment, null = 1
-  const uint4* tiles;      // {expert, c0, c1, 0}; null = dense tiles of TM rows
-  const uint32_t* n_tiles;
-  uint32_t rows;           // dense: number of rows
-  int N, K;                // output rows per matrix, reduction length
-  uint16_t* h_out;         // two matrices: f16 SwiGLU rows [*, N] (k order as xin)
-  float* y_out;            // one matrix: fp32 rows [*, N]
-};
-
 template <int TM>
 constexpr size_t gemm_lds_bytes() {
   return size_t(2) * TM * kLdsPitch * 2;
@@ -340,7 +300,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GemmOc
     src[j] = nullptr;
     if (c < c1) {
       const uint32_t a = p.sorted ? p.sorted[c] : c;
-      src[j] = p.xin + size_t(a / p.in_div) * K + 8 * pc;
+      src[j] = p.xin + size_t(a / p.in_div) * f16_pitch(K) + 8 * pc;
     }
   }
   uint4 xv[NB];
@@ -440,7 +400,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GemmOc
         // rows r0 .. r0 + 3 stored in the k order 0 2 1 3 of the next GEMM
         const half2v lo = {(_Float16)h[0], (_Float16)h[2]};
         const half2v hi = {(_Float16)h[1], (_Float16)h[3]};
-        *reinterpret_cast<uint2*>(p.h_out + size_t(a) * p.N + r0) = make_uint2(as_u32(lo), as_u32(hi));
+        *reinterpret_cast<uint2*>(p.h_out + size_t(a) * f16_pitch(p.N) + r0) = make_uint2(as_u32(lo), as_u32(hi));
       } else {
         *reinterpret_cast<float4*>(p.y_out + size_t(a) * p.N + r0) =
             make_float4(acc0[tb][4 * g4], acc0[tb][4 * g4 + 1], acc0[tb][4 * g4 + 2],
@@ -714,7 +674,7 @@ __global__ void __launch_bounds__(64 * (SPL ? 2 * WR : WR * WT))
     src[q] = nullptr;
     if (row < TM && cc < c1) {
       const uint32_t a = p.sorted ? p.sorted[cc] : cc;
-      src[q] = p.xin + size_t(a / p.in_div) * K + 8 * (c % XPR);
+      src[q] = p.xin + size_t(a / p.in_div) * f16_pitch(K) + 8 * (c % XPR);
     }
   }
   // token pieces of step t (XU: of step group t) sit in register slot
@@ -890,7 +850,7 @@ __global__ void __launch_bounds__(64 * (SPL ? 2 * WR : WR * WT))
           h[r] = silu(acc0[tb][4 * g4 + r]) * acc1[tb][4 * g4 + r] * wa;
         const half2v lo = {(_Float16)h[0], (_Float16)h[2]};
         const half2v hi = {(_Float16)h[1], (_Float16)h[3]};
-        *reinterpret_cast<uint2*>(p.h_out + size_t(a) * p.N + r0) = make_uint2(as_u32(lo), as_u32(hi));
+        *reinterpret_cast<uint2*>(p.h_out + size_t(a) * f16_pitch(p.N) + r0) = make_uint2(as_u32(lo), as_u32(hi));
       } else {
         *reinterpret_cast<float4*>(p.y_out + size_t(a) * p.N + r0) =
             make_float4(acc0[tb][4 * g4], acc0[tb][4 * g4 + 1], acc0[tb][4 * g4 + 2],
@@ -906,24 +866,39 @@ __global__ void __launch_bounds__(64 * (SPL ? 2 * WR : WR * WT))
 // (dispatch_scan with a PlanOut, routing_dev.hpp).
 
 // Upper bounds of the tile lists (grid heights): a 128-row tile covers at
-// least 65 rows, the 64- and 32-row lists hold at most one tile per expert.
+// least 65 rows, the 64- and 32-row lists hold at most one tile per expert,
+// the 16-row list one per 16 rows when it is the only one.
 size_t bound128(size_t A, size_t E) { return A / 65 + 1; }
 size_t bound_small(size_t A, size_t E) { return std::min(E, A) + 1; }
+size_t bound16(size_t A, size_t E) {
+  return bound_small(A, E) + (prefill_narrow(A, E) ? A / 16 : 0);
+}
 
 // ----------------------------------------------------------- conversions
 
-// x -> f16 with the k order 0 2 1 3 4 6 5 7 inside every group of eight.
+// x -> f16 with the k order 0 2 1 3 4 6 5 7 inside every group of eight, and
+// the group sums behind the row.
 template <typename XT>
 __global__ void __launch_bounds__(256)
-    to_f16_kernel(const XT* __restrict__ x, size_t n8, uint4* __restrict__ out) {
-  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+    to_f16_kernel(const XT* __restrict__ x, uint32_t n8, uint32_t K8, uint4* __restrict__ out) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i >= n8) return;
   float v[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = to_f32(x[8 * i + j]);
+  for (int j = 0; j < 8; ++j) v[j] = to_f32(x[8 * size_t(i) + j]);
   const half2v a = {(_Float16)v[0], (_Float16)v[2]}, b = {(_Float16)v[1], (_Float16)v[3]};
   const half2v c = {(_Float16)v[4], (_Float16)v[6]}, d = {(_Float16)v[5], (_Float16)v[7]};
-  out[i] = make_uint4(as_u32(a), as_u32(b), as_u32(c), as_u32(d));
+  const uint32_t r = i / K8, c8 = i - r * K8;
+  const size_t K = 8 * size_t(K8);
+  uint4* row = out + r * (f16_pitch(K) / 8);
+  row[c8] = make_uint4(as_u32(a), as_u32(b), as_u32(c), as_u32(d));
+  // the group of 16 with the neighbouring thread (K8 is even)
+  float t = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) t += (float)(_Float16)v[j];
+  t += __shfl_xor(t, 1, kWave);
+  const int term = int(c8 & 1u);
+  reinterpret_cast<uint16_t*>(row)[f16_sum_at(K, c8 / 2, term)] = f16_sum_term(t, term);
 }
 
 // out = (residual + ys) + y ranks 0..k-1 of the token, in that order; one
@@ -1114,8 +1089,9 @@ struct PlanView {
   uint4* l128;
   uint4* l64;
   uint4* l32;
+  uint4* l16;
   uint32_t* counts;
-  size_t n128, n64, n32;
+  size_t n128, n64, n32, n16;
 };
 
 PlanView plan_view(uint32_t* plan, size_t A, size_t E) {
@@ -1123,29 +1099,80 @@ PlanView plan_view(uint32_t* plan, size_t A, size_t E) {
   v.n128 = bound128(A, E);
   v.n64 = bound_small(A, E);
   v.n32 = bound_small(A, E);
+  v.n16 = bound16(A, E);
   v.l128 = reinterpret_cast<uint4*>(plan);
   v.l64 = v.l128 + v.n128;
   v.l32 = v.l64 + v.n64;
-  v.counts = reinterpret_cast<uint32_t*>(v.l32 + v.n32);
+  v.l16 = v.l32 + v.n32;
+  v.counts = reinterpret_cast<uint32_t*>(v.l16 + v.n16);
   return v;
 }
 
-// The three tile-list launches of one GEMM.
+// True when the LDS DMA can stage the GEMM's operands: matrices aligned to
+// the piece it moves per lane, whole workgroups of rows, and input rows
+// within the 32-bit offset of a lane.
+bool wave_gemm_takes(int quant, const GemmArgs& a) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(a.w0) | reinterpret_cast<uintptr_t>(a.w1);
+  return p % (quant == INFERNO_Q4_K ? 16 : 4) == 0 && a.N % 256 == 0 &&
+         a.in_rows * f16_pitch(a.K) * 2 <= size_t(0xffffffffu);
+}
+
+template <int Q, int NMAT, int RB, int NB, int OCC>
+int launch_wave_gemm(hipStream_t s, const GemmArgs& a, unsigned grid_y) {
+  constexpr size_t lds = grouped::lds_bytes<Q, NMAT, RB, NB>();
+  auto kern = grouped::wave_gemm_kernel<Q, NMAT, RB, NB, OCC>;
+  static_assert(lds <= 64 * 1024, "within the default dynamic LDS limit");
+  const dim3 grid(unsigned(a.N / (16 * RB * grouped::kWaves)), grid_y);
+  kern<<<grid, 256, lds, s>>>(a);
+  INF_LAUNCHED();
+  return INFERNO_OK;
+}
+
+template <int NMAT, int NB, int OCC>
+int launch_wave_q(hipStream_t s, int quant, const GemmArgs& a, unsigned grid_y) {
+  constexpr int RB = NMAT == 2 ? 1 : 2;
+  switch (quant) {
+    case INFERNO_Q2_K: return launch_wave_gemm<INFERNO_Q2_K, NMAT, RB, NB, OCC>(s, a, grid_y);
+    case INFERNO_Q3_K: return launch_wave_gemm<INFERNO_Q3_K, NMAT, RB, NB, OCC>(s, a, grid_y);
+    case INFERNO_Q4_K: return launch_wave_gemm<INFERNO_Q4_K, NMAT, RB, NB, OCC>(s, a, grid_y);
+    case INFERNO_Q6_K:
+      if constexpr (NMAT == 1) return launch_wave_gemm<INFERNO_Q6_K, 1, 2, NB, OCC>(s, a, grid_y);
+      break;
+  }
+  set_error("quant kind has no grouped GEMM");
+  return INFERNO_ERR_INVALID;
+}
+
+// The tile-list launches of one GEMM.
 // A list no expert can fill (max_rows rows at most: no 128-row tile below
 // 65 rows, no 64-row tile below 33) is not launched; its grid of workgroups
-// that find no tile would still take a few microseconds.
+// that find no tile would still take a few microseconds. wave: the DMA
+// kernels take the operands; they run the tiles of up to 64 rows (measured in
+// grouped_gemm.hpp; at 128 rows the matrix cores and not the loads are the
+// longer part, and the kernels above keep them).
 template <int NMAT>
-int launch_tiled(hipStream_t s, int quant, GemmArgs a, const PlanView& v, size_t max_rows) {
+int launch_tiled(hipStream_t s, int quant, GemmArgs a, const PlanView& v, size_t max_rows,
+                 bool narrow, bool wave) {
   int st;
-  a.tiles = v.l128;
-  a.n_tiles = v.counts;
-  if (max_rows > 64 && (st = launch_gemm_q<NMAT, 128>(s, quant, a, unsigned(v.n128)))) return st;
-  a.tiles = v.l64;
-  a.n_tiles = v.counts + 1;
-  if (max_rows > 32 && (st = launch_gemm_q<NMAT, 64>(s, quant, a, unsigned(v.n64)))) return st;
-  a.tiles = v.l32;
-  a.n_tiles = v.counts + 2;
-  return launch_gemm_q<NMAT, 32>(s, quant, a, unsigned(v.n32));
+  if (!narrow) {
+    a.tiles = v.l128;
+    a.n_tiles = v.counts;
+    if (max_rows > 64 && (st = launch_gemm_q<NMAT, 128>(s, quant, a, unsigned(v.n128)))) return st;
+    a.tiles = v.l64;
+    a.n_tiles = v.counts + 1;
+    if (max_rows > 32 && (st = wave ? launch_wave_q<NMAT, 4, 3>(s, quant, a, unsigned(v.n64))
+                                    : launch_gemm_q<NMAT, 64>(s, quant, a, unsigned(v.n64))))
+      return st;
+    a.tiles = v.l32;
+    a.n_tiles = v.counts + 2;
+    if (max_rows > 16 && (st = wave ? launch_wave_q<NMAT, 2, 4>(s, quant, a, unsigned(v.n32))
+                                    : launch_gemm_q<NMAT, 32>(s, quant, a, unsigned(v.n32))))
+      return st;
+  }
+  a.tiles = v.l16;
+  a.n_tiles = v.counts + 3;
+  return wave ? launch_wave_q<NMAT, 1, 4>(s, quant, a, unsigned(v.n16))
+              : launch_gemm_q<NMAT, 32>(s, quant, a, unsigned(v.n16));
 }
 
 // Dense Q8_0 GEMM over a small batch with 32 weight rows per workgroup (one
@@ -1200,27 +1227,68 @@ bool prefill_dense_supported(int quant, int down_quant, size_t H, size_t Is) {
 
 PlanOut prefill_plan_out(uint32_t* plan, size_t A, size_t E) {
   const PlanView v = plan_view(plan, A, E);
-  return PlanOut{v.l128, v.l64, v.l32, v.counts};
+  return PlanOut{v.l128, v.l64, v.l32, v.l16, v.counts, prefill_narrow(A, E)};
 }
 
 size_t prefill_plan_words(size_t A, size_t E) {
-  return 4 * (bound128(A, E) + 2 * bound_small(A, E)) + 4;
+  return 4 * (bound128(A, E) + 2 * bound_small(A, E) + bound16(A, E)) + 4;
 }
 
 int launch_to_f16(hipStream_t s, const void* x, int x_dtype, size_t rows, size_t K,
                   uint16_t* out) {
   const size_t n8 = rows * K / 8;
   if (n8 == 0) return INFERNO_OK;
+  if (n8 > 0xffffffffu || K % kUnit) {
+    set_error("f16 conversion: rows of a multiple of 256, rows * K / 8 < 2^32");
+    return INFERNO_ERR_INVALID;
+  }
   const unsigned grid = unsigned((n8 + 255) / 256);
+  const uint32_t N8 = uint32_t(n8), K8 = uint32_t(K / 8);
   if (x_dtype == INFERNO_BF16)
-    to_f16_kernel<uint16_t><<<grid, 256, 0, s>>>(static_cast<const uint16_t*>(x), n8,
+    to_f16_kernel<uint16_t><<<grid, 256, 0, s>>>(static_cast<const uint16_t*>(x), N8, K8,
                                                  reinterpret_cast<uint4*>(out));
   else
-    to_f16_kernel<float><<<grid, 256, 0, s>>>(static_cast<const float*>(x), n8,
+    to_f16_kernel<float><<<grid, 256, 0, s>>>(static_cast<const float*>(x), N8, K8,
                                               reinterpret_cast<uint4*>(out));
   INF_LAUNCHED();
   return INFERNO_OK;
 }
+
+namespace {
+GemmArgs gate_up_args(const PrefillRouted& p) {
+  GemmArgs g{};
+  g.w0 = static_cast<const uint8_t*>(p.gate);
+  g.w1 = static_cast<const uint8_t*>(p.up);
+  g.stride = p.I * (p.H / kUnit) * size_t(block_bytes(p.quant));
+  g.xin = p.x16;
+  g.in_div = uint32_t(p.k);
+  g.in_rows = p.T;
+  g.sorted = p.sorted;
+  g.route_w = p.weights;
+  g.N = int(p.I);
+  g.K = int(p.H);
+  g.h_out = p.h16;
+  return g;
+}
+GemmArgs down_args(const PrefillRouted& p) {
+  GemmArgs d{};
+  d.w0 = static_cast<const uint8_t*>(p.down);
+  d.stride = p.H * (p.I / kUnit) * size_t(block_bytes(p.down_quant));
+  d.xin = p.h16;
+  d.in_div = 1;
+  d.in_rows = p.T * p.k;
+  d.sorted = p.sorted;
+  d.N = int(p.H);
+  d.K = int(p.I);
+  d.y_out = p.y;
+  return d;
+}
+// Both GEMMs of the layer take the DMA kernels or neither does: the down reads
+// the group sums that the gate/up writes.
+bool wave_layer(const PrefillRouted& p) {
+  return wave_gemm_takes(p.quant, gate_up_args(p)) && wave_gemm_takes(p.down_quant, down_args(p));
+}
+}  // namespace
 
 int launch_prefill_gate_up(hipStream_t s, const PrefillRouted& p) {
   const size_t A = p.T * p.k;
@@ -1229,35 +1297,15 @@ int launch_prefill_gate_up(hipStream_t s, const PrefillRouted& p) {
     set_error("MFMA prefill path does not cover this layer");
     return INFERNO_ERR_INVALID;
   }
-  const PlanView v = plan_view(p.plan, A, p.E);
-  GemmArgs g{};
-  g.w0 = static_cast<const uint8_t*>(p.gate);
-  g.w1 = static_cast<const uint8_t*>(p.up);
-  g.stride = p.I * (p.H / kUnit) * size_t(block_bytes(p.quant));
-  g.xin = p.x16;
-  g.in_div = uint32_t(p.k);
-  g.sorted = p.sorted;
-  g.route_w = p.weights;
-  g.N = int(p.I);
-  g.K = int(p.H);
-  g.h_out = p.h16;
-  return launch_tiled<2>(s, p.quant, g, v, p.max_rows ? p.max_rows : A);
+  return launch_tiled<2>(s, p.quant, gate_up_args(p), plan_view(p.plan, A, p.E),
+                         p.max_rows ? p.max_rows : A, prefill_narrow(A, p.E), wave_layer(p));
 }
 
 int launch_prefill_down(hipStream_t s, const PrefillRouted& p) {
   const size_t A = p.T * p.k;
   if (A == 0) return INFERNO_OK;
-  const PlanView v = plan_view(p.plan, A, p.E);
-  GemmArgs d{};
-  d.w0 = static_cast<const uint8_t*>(p.down);
-  d.stride = p.H * (p.I / kUnit) * size_t(block_bytes(p.down_quant));
-  d.xin = p.h16;
-  d.in_div = 1;
-  d.sorted = p.sorted;
-  d.N = int(p.H);
-  d.K = int(p.I);
-  d.y_out = p.y;
-  return launch_tiled<1>(s, p.down_quant, d, v, p.max_rows ? p.max_rows : A);
+  return launch_tiled<1>(s, p.down_quant, down_args(p), plan_view(p.plan, A, p.E),
+                         p.max_rows ? p.max_rows : A, prefill_narrow(A, p.E), wave_layer(p));
 }
 
 int launch_prefill_dense(hipStream_t s, int quant, int down_quant, const void* gate,

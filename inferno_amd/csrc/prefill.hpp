@@ -24,20 +24,49 @@ size_t prefill_plan_words(size_t A, size_t E);
 // The tile lists inside that scratch, for the dispatch launch to fill
 // (launch_dispatch with a plan) before launch_prefill_gate_up reads them.
 PlanOut prefill_plan_out(uint32_t* plan, size_t A, size_t E);
+// True when a batch of A assignments over E experts takes 16-row tiles only.
+// One launch per GEMM instead of one per tile size that an expert could
+// fill; an expert of more rows reads its weights once per 16 (of which L2 and
+// the Infinity Cache hold the later ones). Up to 10 rows per expert on average:
+// 16 caller-routed tokens x 8 over 64 experts (2 rows each) 61 -> 52 us, 64
+// tokens (8 rows) 125 -> 118 us; 32 tokens x 10 over 128 experts even.
+constexpr size_t kNarrowRows = 10;
+inline bool prefill_narrow(size_t A, size_t E) { return A <= kNarrowRows * E; }
 
-// x [rows, K] (bf16 or fp32) -> f16 [rows, K], round to nearest even.
+// Halfs per row of the f16 activations the grouped GEMMs read (x16, h16): K
+// values, the sums of every 16 of them in two f16 terms (K / 8 halfs: per 256
+// values 16 first terms, then 16 second ones, in the k order of the values),
+// and 128 bytes of padding: a tile reads the same 128 bytes of up to 128 rows
+// at once, and rows of a multiple of 512 bytes apart put all of them on one
+// or two of the 16 L2 channels.
+HD constexpr size_t f16_pitch(size_t K) { return K + K / 8 + 64; }
+// Where a row of K values holds term `term` (0 or 1) of the sum of its
+// group-th 16 values.
+HD constexpr size_t f16_sum_at(size_t K, size_t group, int term) {
+  return K + 32 * (group / 16) + 16 * size_t(term) +
+         ((group & 12) | ((group & 1) << 1) | ((group >> 1) & 1));
+}
+// The two terms of a group sum t: t / 16 (never past f16's range, as the
+// values are not) rounded to f16, and the rest times 2^11.
+__device__ __forceinline__ uint16_t f16_sum_term(float t, int term) {
+  const float m = t * 0.0625f;
+  const _Float16 hi = (_Float16)m;
+  return __builtin_bit_cast(uint16_t, term == 0 ? hi : (_Float16)((m - (float)hi) * 2048.0f));
+}
+
+// x [rows, K] (bf16 or fp32) -> f16 rows of f16_pitch(K), round to nearest even.
 int launch_to_f16(hipStream_t s, const void* x, int x_dtype, size_t rows, size_t K, uint16_t* out);
 
 struct PrefillRouted {
   int quant, down_quant;
   const void *gate, *up, *down;  // packed experts [E][rows][blocks]
-  const uint16_t* x16;           // [T, H] f16
+  const uint16_t* x16;           // [T] f16 rows of f16_pitch(H)
   const uint32_t* offsets;       // [E+1] from the dispatch
   const uint32_t* sorted;        // [A]
   const uint32_t* active;        // [E+1]
   const float* weights;          // [A] routing weights (folded into h)
   size_t T, k, E, H, I;
-  uint16_t* h16;                 // [A, I] SwiGLU intermediate, f16
+  uint16_t* h16;                 // [A] f16 rows of f16_pitch(I): SwiGLU intermediate
   float* y;                      // [A, H] per-assignment down rows
   uint32_t* plan;                // prefill_plan_words(A, E)
   // most rows one expert can take: T when every token's ids are distinct

@@ -10,6 +10,7 @@
 // (routing_dev.hpp).
 #include <cstdlib>
 
+#include "prefill.hpp"
 #include "routing_dev.hpp"
 
 namespace inferno {
@@ -183,8 +184,14 @@ __global__ void __launch_bounds__(256)
           return uint32_t(__builtin_bit_cast(uint16_t, (_Float16)lo)) |
                  (uint32_t(__builtin_bit_cast(uint16_t, (_Float16)hi)) << 16);
         };
-        *reinterpret_cast<uint4*>(x16 + size_t(t0 + 16 * b + r) * H + k0 + 8 * g) =
+        uint16_t* row = x16 + size_t(t0 + 16 * b + r) * f16_pitch(H);
+        *reinterpret_cast<uint4*>(row + k0 + 8 * g) =
             make_uint4(pair(v[0], v[2]), pair(v[1], v[3]), pair(v[4], v[6]), pair(v[5], v[7]));
+        float sum = 0.f;  // of the group of 16 with the lane of the neighbouring g
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum += (float)(_Float16)v[j];
+        sum += __shfl_xor(sum, 16, kWave);
+        row[f16_sum_at(H, (k0 + 8 * g) / 16, g & 1)] = f16_sum_term(sum, g & 1);
       }
     }
   }
@@ -310,9 +317,15 @@ __global__ void __launch_bounds__(256 * KS)
         h[2 * i] = f16(u.xv[b][i] << 16);
         h[2 * i + 1] = f16(u.xv[b][i] & 0xffff0000u);
       }
-      *reinterpret_cast<uint4*>(x16 + size_t(t) * H + kb * 32 + 8 * g) =
+      uint16_t* row = x16 + size_t(t) * f16_pitch(H);
+      *reinterpret_cast<uint4*>(row + kb * 32 + 8 * g) =
           make_uint4(h[0] | (h[2] << 16), h[1] | (h[3] << 16), h[4] | (h[6] << 16),
                      h[5] | (h[7] << 16));
+      float sum = 0.f;  // of the group of 16 with the lane of the neighbouring g
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sum += (float)__builtin_bit_cast(_Float16, uint16_t(h[j]));
+      sum += __shfl_xor(sum, 16, kWave);
+      row[f16_sum_at(H, kb * 2 + g / 2, g & 1)] = f16_sum_term(sum, g & 1);
     }
   };
   // the host launches this kernel only when 2 * KS divides the chunk's blocks

@@ -369,18 +369,21 @@ __device__ __forceinline__ int expert_bits(int E) {
 }
 
 // Tiles of one expert with n rows: full 128-row tiles, then the remainder r
-// as one 128-row (r > 64), 64-row (r > 32) or 32-row tile. The
+// as one 128-row (r > 64), 64-row (r > 32), 32-row (r > 16) or 16-row tile. The
 // dequantisation cost of a tile does not depend on its row count, the MFMA
 // cost does: small remainders take the cheaper narrow tiles.
 struct TileCounts {
-  uint32_t t128, t64, t32;
+  uint32_t t128, t64, t32, t16;
 };
-__device__ __forceinline__ TileCounts tile_counts(uint32_t n) {
+// narrow: 16-row tiles only (one launch; batches of few rows per expert).
+__device__ __forceinline__ TileCounts tile_counts(uint32_t n, bool narrow) {
+  if (narrow) return TileCounts{0, 0, 0, (n + 15) / 16};
   const uint32_t r = n % 128;
-  TileCounts t{n / 128, 0, 0};
+  TileCounts t{n / 128, 0, 0, 0};
   if (r > 64) t.t128 += 1;
   else if (r > 32) t.t64 = 1;
-  else if (r > 0) t.t32 = 1;
+  else if (r > 16) t.t32 = 1;
+  else if (r > 0) t.t16 = 1;
   return t;
 }
 
@@ -433,26 +436,28 @@ __device__ __forceinline__ void dispatch_scan(const uint32_t* count, int E, uint
   }
   if (!write || plan.l128 == nullptr) return;  // uniform
   TileCounts t4[4];
-  uint32_t s128 = 0, s64 = 0, s32 = 0;
+  uint32_t s128 = 0, s64 = 0, s32 = 0, s16 = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    t4[j] = tile_counts(c4[j]);  // zero for e >= E (c4 is zero there)
+    t4[j] = tile_counts(c4[j], plan.narrow);  // zero for e >= E (c4 is zero there)
     s128 += t4[j].t128;
     s64 += t4[j].t64;
     s32 += t4[j].t32;
+    s16 += t4[j].t16;
   }
-  uint32_t i128 = s128, i64 = s64, i32 = s32;  // inclusive wave scans
+  uint32_t i128 = s128, i64 = s64, i32 = s32, i16 = s16;  // inclusive wave scans
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const uint32_t a = __shfl_up(i128, o, kWave), b = __shfl_up(i64, o, kWave),
-                   c = __shfl_up(i32, o, kWave);
+                   c = __shfl_up(i32, o, kWave), d = __shfl_up(i16, o, kWave);
     if (lane >= o) {
       i128 += a;
       i64 += b;
       i32 += c;
+      i16 += d;
     }
   }
-  uint32_t o128 = i128 - s128, o64 = i64 - s64, o32 = i32 - s32, lo = c_first;
+  uint32_t o128 = i128 - s128, o64 = i64 - s64, o32 = i32 - s32, o16 = i16 - s16, lo = c_first;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const uint32_t e = uint32_t(4 * lane + j), hi = lo + c4[j];
@@ -460,15 +465,21 @@ __device__ __forceinline__ void dispatch_scan(const uint32_t* count, int E, uint
       plan.l128[o128 + q] = make_uint4(e, lo + 128 * q, min(hi, lo + 128 * (q + 1)), 0);
     if (t4[j].t64) plan.l64[o64] = make_uint4(e, lo + 128 * t4[j].t128, hi, 0);
     if (t4[j].t32) plan.l32[o32] = make_uint4(e, lo + 128 * t4[j].t128, hi, 0);
+    for (uint32_t q = 0; q < t4[j].t16; ++q) {  // one, unless narrow
+      const uint32_t at = lo + 128 * t4[j].t128 + 16 * q;
+      plan.l16[o16 + q] = make_uint4(e, at, min(hi, at + 16), 0);
+    }
     o128 += t4[j].t128;
     o64 += t4[j].t64;
     o32 += t4[j].t32;
+    o16 += t4[j].t16;
     lo = hi;
   }
   if (lane == 63) {
     plan.counts[0] = i128;
     plan.counts[1] = i64;
     plan.counts[2] = i32;
+    plan.counts[3] = i16;
   }
 }
 

@@ -1,0 +1,94 @@
+"""The grouped GEMM's DMA kernels (inferno_amd/csrc/grouped_gemm.hpp): source
+addresses of the weight copies (CPU, tests/weight_dma_check.hip replays the
+kernel's own offsets), and on the GPU the tile edges (15, 16, 17, 32, 33, 63,
+64, 65 rows of one expert beside experts of 0, 1 and 2 rows), odd and even
+super-block counts, every format pair, and weights that the DMA cannot take."""
+import os
+import shutil
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as orc
+from inferno_amd import Q2_K, Q3_K, Q4_K, Q6_K, ops
+
+ROOT = Path(__file__).resolve().parent.parent
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+def test_weight_dma_addresses(tmp_path):
+    if not (Path(HIPCC).exists() or shutil.which(HIPCC)):
+        pytest.skip("hipcc not found")
+    exe = tmp_path / "dmacheck"
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O1", "-std=c++17", f"-I{ROOT / 'include'}",
+                    f"-I{ROOT / 'inferno_amd' / 'csrc'}", str(ROOT / "tests" / "weight_dma_check.hip"),
+                    "-o", str(exe)], check=True, capture_output=True, text=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout.startswith("OK "), r.stdout[-2000:] + r.stderr
+
+
+def _ids(rows, E):
+    """One expert per assignment (k = 1): expert e takes rows[e] tokens, shuffled."""
+    ids = np.concatenate([np.full(n, e) for e, n in enumerate(rows)]).astype(np.uint32)
+    return np.random.default_rng(3).permutation(ids)
+
+
+def _run(quant, down, H, I, rows, bf16, shift=0):
+    dev = torch.device("cuda:0")
+    E = len(rows)
+    ids = _ids(rows, E)
+    T = len(ids)
+    mats = [ops.synth_quantized(q, 5 + i, 0.02, E * r, c, dev)
+            for i, (q, r, c) in enumerate(((quant, I, H), (quant, I, H), (down, H, I)))]
+    placed = []
+    for m in mats:  # the same bytes at an address that is `shift` past an aligned one
+        buf = torch.empty(m.numel() + 16, dtype=torch.uint8, device=dev)
+        buf[shift:shift + m.numel()] = m
+        placed.append(buf[shift:shift + m.numel()])
+    g = torch.Generator(device=dev).manual_seed(7)
+    x = torch.randn(T, H, generator=g, device=dev)
+    x = x.bfloat16() if bf16 else x
+    w = torch.rand(T, generator=g, device=dev) + 0.5
+    args = (quant, down, *placed, x, torch.from_numpy(ids.view(np.int32)).to(dev), w, 1, E, I)
+    out = ops.gguf_moe(*args)
+    again = ops.gguf_moe(*args)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    ref = orc.moe_routed(quant, down, *(m.cpu().numpy() for m in mats), x.float().cpu().numpy(),
+                         ids, w.cpu().numpy(), E, 1, I)
+    got = out.cpu().numpy()
+    return float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+
+
+# h is rounded to f16 and so are fp32 tokens (2^-12 of a value each, at random);
+# Q6_K weights too: 2e-3 is the bound of the layers' own tests
+BOUND = 2e-3
+PAIRS = [(Q2_K, Q2_K), (Q3_K, Q3_K), (Q4_K, Q4_K), (Q4_K, Q6_K), (Q2_K, Q3_K)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,down", PAIRS)
+@pytest.mark.parametrize("H,I", [(512, 512), (768, 256), (256, 768)])
+@pytest.mark.parametrize("rows", [(15, 0, 16, 17), (32, 33, 1, 0), (63, 2, 64, 65)],
+                         ids=["to16", "to32", "to64"])
+def test_tile_edges(quant, down, H, I, rows):
+    assert _run(quant, down, H, I, rows, bf16=True) < BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,down", PAIRS)
+def test_sixteen_row_tiles_only(quant, down):
+    # 70 rows over 9 experts: the batch takes 16-row tiles only, the first
+    # expert two of them
+    assert _run(quant, down, 512, 512, (20, 16, 15, 8, 5, 3, 2, 1, 0), bf16=False) < BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,down", PAIRS)
+@pytest.mark.parametrize("shift", [2, 4])
+def test_weights_at_any_address(quant, down, shift):
+    # 2 bytes past a word (and 4 past 16 bytes for Q4_K): not the DMA's rows
+    assert _run(quant, down, 512, 256, (18, 30, 4, 0), bf16=True, shift=shift) < BOUND
