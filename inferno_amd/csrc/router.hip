@@ -413,17 +413,18 @@ static bool bf16x3_enabled() {
 
 // K chunks for the router logits of a T-token batch (bf16 tokens on the
 // bf16x3 kernel, fp32 tokens on the fp32 MFMA kernel): 1 when the
-// batch alone gives the kernel enough workgroups; else the most (a power of
-// two, up to kMaxRouterParts) that keeps at most kRouterSplitGroups
-// workgroups of the one-group kernel and a whole number of 32-deep block
-// pairs per chunk.
+// batch alone gives the kernel enough workgroups; else the most (up to
+// kMaxRouterParts) that keeps at most kRouterSplitGroups workgroups of the
+// one-group kernel and a whole number of 32-deep block pairs per chunk. Any
+// divisor of the pairs: H 2816 takes 11 chunks (a power of two gave it 4 and
+// the launch 15.4 us instead of 7.3).
 constexpr size_t kRouterSplitGroups = 256;
 int router_logit_parts_max(size_t T, size_t H, size_t E) {
   if (H % 256) return 1;
   const size_t base = ((E + 63) / 64) * ((T + 15) / 16);
   if (base * 2 > kRouterSplitGroups) return 1;
-  int z = 1;
-  while (z < kMaxRouterParts && base * size_t(2 * z) <= kRouterSplitGroups && (H / 32) % size_t(4 * z) == 0) z *= 2;
+  int z = kMaxRouterParts;
+  while (z > 1 && (base * size_t(z) > kRouterSplitGroups || (H / 64) % size_t(z) != 0)) --z;
   return z;
 }
 bool router_writes_x16(size_t T, size_t H, size_t E, int x_dtype, int parts) {
