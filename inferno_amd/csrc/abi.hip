@@ -2,12 +2,14 @@
 // Err paths, e.g. crates/backend/src/metal/gguf_moe.rs:84-121 and
 // crates/backend/src/metal/moe.rs:582-623), workspace carving and kernel
 // sequencing. No function allocates device memory or synchronises.
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <string>
 #include <vector>
 
 #include "decode.hpp"
+#include "dense_q8.hpp"
 #include "prefill.hpp"
 #include "timing.hpp"
 #include "gemv_common.hpp"
@@ -381,6 +383,23 @@ int inferno_q8_0_gate_up_swiglu(void* stream, const void* gate, size_t gate_byte
   if ((st = need_ws(workspace, workspace_bytes, gemv_stage_bytes(INFERNO_Q8_0, T, H, x_dtype))))
     return st;
   if (int st_ = require_device()) return st_;
+  if (dense_q8_takes(T, gate, up, workspace)) {
+    DenseQ8 p{};
+    p.w0 = gate;
+    p.w1 = up;
+    p.x = static_cast<uint16_t*>(workspace);
+    p.terms = x_dtype == INFERNO_BF16 ? 1 : 2;
+    p.pitch = dense_q8_pitch(H, p.terms);
+    p.scaled = true;
+    p.T = T;
+    p.K = H;
+    p.N = Is;
+    p.out = out;
+    if ((st = launch_dense_q8_stage(as_stream(stream), x, x_dtype, T, H,
+                                    static_cast<uint16_t*>(workspace))))
+      return st;
+    return launch_dense_q8(as_stream(stream), p);
+  }
   return launch_gemv_gate_up_dense(as_stream(stream), INFERNO_Q8_0, gate, up, x, x_dtype,
                                    static_cast<uint32_t*>(workspace), false, T, H, Is, out,
                                    nullptr);
@@ -399,6 +418,24 @@ int inferno_q8_0_matvec_add2(void* stream, const void* w, size_t w_bytes, const 
   if ((st = need_ws(workspace, workspace_bytes, gemv_stage_bytes(INFERNO_Q8_0, T, In, INFERNO_F32))))
     return st;
   if (int st_ = require_device()) return st_;
+  if (dense_q8_takes(T, w, nullptr, workspace)) {
+    DenseQ8 p{};
+    p.w0 = w;
+    p.x = static_cast<uint16_t*>(workspace);
+    p.terms = 2;
+    p.pitch = dense_q8_pitch(In, 2);
+    p.scaled = true;
+    p.T = T;
+    p.K = In;
+    p.N = O;
+    p.out = out;
+    p.res_a = residual_a;
+    p.res_b = residual_b;
+    if ((st = launch_dense_q8_stage(as_stream(stream), input, INFERNO_F32, T, In,
+                                    static_cast<uint16_t*>(workspace))))
+      return st;
+    return launch_dense_q8(as_stream(stream), p);
+  }
   return launch_gemv_down_dense(as_stream(stream), INFERNO_Q8_0, w, input,
                                 static_cast<uint32_t*>(workspace), false, nullptr, 0, residual_a,
                                 residual_b, T, In, O, out);
@@ -592,11 +629,37 @@ bool layer_takes_decode(const inferno_moe_layer* L, size_t T, int x_dtype) {
   const int sdq = L->shared_down_quant ? L->shared_down_quant : INFERNO_Q8_0;
   const bool shared_q8 = Is == 0 || (sq == INFERNO_Q8_0 && sdq == INFERNO_Q8_0);
   if (layer_shared_slot(L, T, x_dtype)) return true;
-  return decode_supported(T, L->top_k, L->experts, L->hidden, L->intermediate, Is, x_dtype,
-                          L->quant, L->down_quant) &&
-         shared_q8 &&
-         (T == 1 || !use_mfma(L->quant, L->down_quant, T, L->top_k, L->experts, L->hidden,
-                              L->intermediate, Is));
+  if (!decode_supported(T, L->top_k, L->experts, L->hidden, L->intermediate, Is, x_dtype,
+                        L->quant, L->down_quant) ||
+      !shared_q8)
+    return false;
+  if (T == 1) return true;
+  const size_t H = L->hidden, I = L->intermediate, k = L->top_k;
+  if (use_mfma(L->quant, L->down_quant, T, k, L->experts, H, I, Is)) return false;
+  // (a threshold given in the environment is the only rule then)
+  return std::getenv("INFERNO_PREFILL_MIN_ASSIGNMENTS") != nullptr ||
+         !prefill_routed_supported(L->quant, L->down_quant, H, I, L->experts) ||
+         !grouped_beats_decode(T * k, H, I,
+                               2 * matrix_bytes(L->quant, I, H) + matrix_bytes(L->down_quant, H, I),
+                               Is != 0);
+}
+
+// True when a layer forward that does not take the decode launches runs its
+// routed experts on the grouped GEMMs: those of decode_supported shapes
+// always do (layer_takes_decode has weighed the two), others from the
+// assignment counts of use_mfma (below them their GEMV kernels keep fp32
+// activations).
+bool layer_takes_grouped(const inferno_moe_layer* L, size_t T, int x_dtype) {
+  const size_t Is = L->shared_intermediate;
+  const int sq = L->shared_quant ? L->shared_quant : INFERNO_Q8_0;
+  const int sdq = L->shared_down_quant ? L->shared_down_quant : INFERNO_Q8_0;
+  const bool shared_q8 = Is == 0 || (sq == INFERNO_Q8_0 && sdq == INFERNO_Q8_0);
+  if (use_mfma(L->quant, L->down_quant, T, L->top_k, L->experts, L->hidden, L->intermediate, Is))
+    return true;
+  return shared_q8 && T > 1 && std::getenv("INFERNO_PREFILL_MIN_ASSIGNMENTS") == nullptr &&
+         prefill_routed_supported(L->quant, L->down_quant, L->hidden, L->intermediate, L->experts) &&
+         decode_supported(T, L->top_k, L->experts, L->hidden, L->intermediate, Is, x_dtype,
+                          L->quant, L->down_quant);
 }
 
 // logits_ready: the tokens' router logits [T, E], already formed (the
@@ -687,7 +750,7 @@ int layer_forward(void* stream, const inferno_moe_layer* L, const void* x, int x
   const bool router_blas = w.rblas != nullptr && w.blas_lib != nullptr &&
                            router_blas_takes(T, H, E, x_dtype);
   const int parts = router_blas ? 1 : router_logit_parts(T, H, E, x_dtype);
-  const bool mfma_path = use_mfma(L->quant, L->down_quant, T, k, E, H, I, Is);
+  const bool mfma_path = layer_takes_grouped(L, T, x_dtype);
   // the shared expert on the dense MFMA GEMMs when its formats have them
   // (Q8_0; the Laguna XS Q4_K gate/up with Q4_K or Q6_K down), else on the
   // GEMV kernels

@@ -30,6 +30,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "dense_q8.hpp"
 #include "grouped_gemm.hpp"
 #include "routing_dev.hpp"
 
@@ -1108,12 +1109,13 @@ PlanView plan_view(uint32_t* plan, size_t A, size_t E) {
   return v;
 }
 
-// True when the LDS DMA can stage the GEMM's operands: matrices aligned to
-// the piece it moves per lane, whole workgroups of rows, and input rows
-// within the 32-bit offset of a lane.
+// True when the LDS DMA can stage the GEMM's operands: matrices and input
+// rows aligned to the piece it moves per lane, whole workgroups of rows, and
+// input rows within the 32-bit offset of a lane.
 bool wave_gemm_takes(int quant, const GemmArgs& a) {
   const uintptr_t p = reinterpret_cast<uintptr_t>(a.w0) | reinterpret_cast<uintptr_t>(a.w1);
   return p % (quant == INFERNO_Q4_K ? 16 : 4) == 0 && a.N % 256 == 0 &&
+         reinterpret_cast<uintptr_t>(a.xin) % 16 == 0 &&
          a.in_rows * f16_pitch(a.K) * 2 <= size_t(0xffffffffu);
 }
 
@@ -1308,6 +1310,14 @@ int launch_prefill_down(hipStream_t s, const PrefillRouted& p) {
                          p.max_rows ? p.max_rows : A, prefill_narrow(A, p.E), wave_layer(p));
 }
 
+// Tokens up to which a layer's Q8_0 shared expert takes the dense Q8_0
+// kernels; above, the library GEMMs on f16 weights expanded per call (their
+// own 12 to 27 us are paid once, their rate is higher). Whole layer, these
+// kernels against the library: H 6144, Is 2048 T = 16 250 / 294 us, 32 332 /
+// 363, 64 412 / 434, 128 535 / 540, 256 799 / 749; H 4096, Is 1536 T = 32 249
+// / 269, 128 310 / 321, 256 485 / 453.
+constexpr size_t kDenseQ8LayerTokens = 128;
+
 int launch_prefill_dense(hipStream_t s, int quant, int down_quant, const void* gate,
                          const void* up, const void* down, const uint16_t* x16, size_t T,
                          size_t H, size_t Is, uint16_t* h16, float* ys, void* blas_ws,
@@ -1316,6 +1326,31 @@ int launch_prefill_dense(hipStream_t s, int quant, int down_quant, const void* g
   if (H % kUnit || Is % kUnit) {
     set_error("MFMA prefill path needs 256-multiple dimensions");
     return INFERNO_ERR_INVALID;
+  }
+  if (quant == INFERNO_Q8_0 && down_quant == INFERNO_Q8_0 && T <= kDenseQ8LayerTokens &&
+      dense_q8_takes(T, gate, up, x16) && dense_q8_takes(T, down, nullptr, h16)) {
+    DenseQ8 g{};
+    g.w0 = gate;
+    g.w1 = up;
+    g.x = x16;
+    g.pitch = f16_pitch(H);
+    g.terms = 1;
+    g.T = T;
+    g.K = H;
+    g.N = Is;
+    g.h16 = h16;
+    g.h_pitch = f16_pitch(Is);
+    if (int st = launch_dense_q8(s, g)) return st;
+    DenseQ8 d{};
+    d.w0 = down;
+    d.x = h16;
+    d.pitch = f16_pitch(Is);
+    d.terms = 1;
+    d.T = T;
+    d.K = Is;
+    d.N = H;
+    d.out = ys;
+    return launch_dense_q8(s, d);
   }
   if (blas_ws != nullptr && lib_ws != nullptr && dense_blas_takes(quant, down_quant, T, H, Is))
     return launch_dense_blas(s, gate, up, down, x16, T, H, Is, ys, blas_ws, lib_ws);

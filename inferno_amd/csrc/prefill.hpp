@@ -18,6 +18,22 @@ bool prefill_routed_supported(int quant, int down_quant, size_t H, size_t I, siz
 // against 1.015, T = 8 1.151 against 1.050, c2 T = 10 0.408 against 0.378).
 constexpr size_t kPrefillMinAssignments = 48;
 constexpr size_t kPrefillMinAssignmentsShared = 66;
+// Several tokens below those counts, in a layer that the fused decode launches
+// also take: the grouped GEMMs when the assignments' expert bytes outweigh
+// their more launches (seven against four, two more with a shared expert).
+// Measured over H 1024 .. 6144, I 512 .. 2048, Q2_K / Q3_K / Q4_K, decode /
+// grouped in us: without a shared expert 2048 x 768 Q4_K 16 assignments 39 /
+// 34, 24 47 / 41; 2816 x 1280 Q2_K 16 48 / 50, 18 51 / 50, 24 61 / 52; 1024 x
+// 512 Q2_K 18 (9 MB) 29 / 29, 32 (17 MB) 33 / 29; with one 4096 x 1536 Q2_K 16
+// (99 MB) 63 / 66, 24 77 / 73, 32 96 / 83; 6144 x 2048 Q2_K 16 (198 MB) 101 /
+// 99, 32 177 / 143; 2048 x 768 Q2_K 32 (50 MB) 44 / 47. A narrow expert under
+// a wide row (6144 x 512: few workgroups, each with a long K) needs more:
+// Q2_K 18 50 / 57, 24 61 / 59, with a shared expert Q4_K 24 64 / 68, 32 78 / 70.
+inline bool grouped_beats_decode(size_t A, size_t H, size_t I, size_t expert_bytes, bool shared) {
+  const bool narrow = H > 4 * I;
+  return shared ? A >= (narrow ? 32 : 16) && A * expert_bytes >= size_t(100) << 20
+                : A >= (narrow ? 24 : 18) && A * expert_bytes >= size_t(14) << 20;
+}
 
 // 32-bit words of the routed planner's scratch (tile lists and counts).
 size_t prefill_plan_words(size_t A, size_t E);

@@ -92,3 +92,66 @@ def test_sixteen_row_tiles_only(quant, down):
 def test_weights_at_any_address(quant, down, shift):
     # 2 bytes past a word (and 4 past 16 bytes for Q4_K): not the DMA's rows
     assert _run(quant, down, 512, 256, (18, 30, 4, 0), bf16=True, shift=shift) < BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 33])
+@pytest.mark.parametrize("H,Is", [(256, 24), (768, 200), (4608, 256)])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_dense_q8_rows(T, H, Is, bf16):
+    # row counts that do not fill a workgroup (8 gate / 8 up rows, 16 rows),
+    # one to 18 K units over four to eight wavefronts, values over 24 binary
+    # orders within a row; the products are fp32-accurate: 1e-5 against fp64
+    dev = torch.device("cuda:0")
+    from inferno_amd import Q8_0
+    g = torch.Generator(device=dev).manual_seed(11)
+    x = torch.randn(T, H, generator=g, device=dev)
+    x = x * torch.exp2(-24 * torch.rand(T, H, generator=g, device=dev)) * 1e3
+    x = x.bfloat16() if bf16 else x
+    wg, wu = (ops.synth_quantized(Q8_0, s, 0.02, Is, H, dev) for s in (1, 2))
+    h = ops.q8_0_gate_up_swiglu(wg, wu, x, Is)
+    a = x.double() @ ops.dequantize(Q8_0, wg).view(Is, H).double().T
+    b = x.double() @ ops.dequantize(Q8_0, wu).view(Is, H).double().T
+    ref = a * torch.sigmoid(a) * b
+    assert float((h - ref).norm() / ref.norm()) < 1e-5
+    O, In = Is, H
+    wd = ops.synth_quantized(Q8_0, 3, 0.02, O, In, dev)
+    inp = torch.randn(T, In, generator=g, device=dev) * 1e-4
+    ra = torch.randn(T, O, generator=g, device=dev) * 1e-5
+    for rb in (None, ra * 0.5):
+        out = ops.q8_0_matvec_add2(wd, inp, ra, rb, O)
+        ref = ra.double() + (0 if rb is None else rb.double()) + \
+            inp.double() @ ops.dequantize(Q8_0, wd).view(O, In).double().T
+        assert float((out - ref).norm() / ref.norm()) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [2, 3, 4, 6])
+@pytest.mark.parametrize("shared", [0, 1024])
+@pytest.mark.parametrize("quant", [Q2_K, Q3_K, Q4_K])
+def test_layer_decode_and_grouped_agree(quant, shared, T, monkeypatch):
+    # both sides of the rule that hands a few tokens to the grouped GEMMs: the
+    # same layer on the fused decode launches (a threshold no batch reaches)
+    # and by the rule, outputs within the rounding of h to f16 (2^-12 each)
+    from inferno_amd import Q8_0, SCORE_SOFTMAX
+    dev = torch.device("cuda:0")
+    H, E, I, k = 3072, 32, 1024, 6
+    mats = [ops.synth_quantized(quant, i, 0.02, E * r, c, dev)
+            for i, (r, c) in enumerate(((I, H), (I, H), (H, I)))]
+    sh = [ops.synth_quantized(Q8_0, 9 + i, 0.02, r, c, dev)
+          for i, (r, c) in enumerate(((1024, H), (1024, H), (H, 1024)))]
+    g = torch.Generator(device=dev).manual_seed(2)
+    layer = ops.MoELayer(
+        hidden=H, experts=E, intermediate=I, top_k=k, quant=quant, down_quant=quant,
+        score_fn=SCORE_SOFTMAX, norm_topk_prob=True, routed_scaling_factor=1.0,
+        router=torch.randn(E, H, generator=g, device=dev) * 0.02, router_bias=None, gate=mats[0],
+        up=mats[1], down=mats[2], shared_intermediate=shared, shared_gate=sh[0], shared_up=sh[1],
+        shared_down=sh[2], max_tokens=T)
+    x = torch.randn(T, H, generator=g, device=dev).bfloat16()
+    by_rule = layer.forward(x)
+    monkeypatch.setenv("INFERNO_PREFILL_MIN_ASSIGNMENTS", "100000")
+    decode = layer.forward(x)
+    monkeypatch.setenv("INFERNO_PREFILL_MIN_ASSIGNMENTS", "1")
+    grouped = layer.forward(x)
+    assert float((by_rule - decode).norm() / decode.norm()) < 2e-3
+    assert float((grouped - decode).norm() / decode.norm()) < 2e-3
