@@ -32,6 +32,7 @@
 
 #include "dense_q8.hpp"
 #include "grouped_gemm.hpp"
+#include "grouped_gemm128.hpp"
 #include "routing_dev.hpp"
 
 namespace inferno {
@@ -1145,13 +1146,39 @@ int launch_wave_q(hipStream_t s, int quant, const GemmArgs& a, unsigned grid_y) 
   return INFERNO_ERR_INVALID;
 }
 
+template <int Q, int NMAT>
+int launch_tile128(hipStream_t s, const GemmArgs& a, unsigned grid_y) {
+  constexpr size_t lds = grouped::lds128_bytes<Q, NMAT>();
+  static_assert(lds <= 80 * 1024, "two workgroups per CU");
+  auto kern = grouped::tile128_gemm_kernel<Q, NMAT>;
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+  INF_HIP(attr);
+  const dim3 grid(unsigned(a.N / (NMAT == 2 ? 128 : 256)), grid_y);
+  kern<<<grid, 256, lds, s>>>(a);
+  INF_LAUNCHED();
+  return INFERNO_OK;
+}
+
+// Tiles of up to 128 rows on the DMA operands. Q6_K (down only) keeps the
+// fragment-load kernel: its two scales per 32 values do not come out of the
+// integer products.
+template <int NMAT>
+int launch_tile128_q(hipStream_t s, int quant, const GemmArgs& a, unsigned grid_y) {
+  switch (quant) {
+    case INFERNO_Q2_K: return launch_tile128<INFERNO_Q2_K, NMAT>(s, a, grid_y);
+    case INFERNO_Q3_K: return launch_tile128<INFERNO_Q3_K, NMAT>(s, a, grid_y);
+    case INFERNO_Q4_K: return launch_tile128<INFERNO_Q4_K, NMAT>(s, a, grid_y);
+  }
+  return launch_gemm_q<NMAT, 128>(s, quant, a, grid_y);
+}
+
 // The tile-list launches of one GEMM.
 // A list no expert can fill (max_rows rows at most: no 128-row tile below
 // 65 rows, no 64-row tile below 33) is not launched; its grid of workgroups
 // that find no tile would still take a few microseconds. wave: the DMA
-// kernels take the operands; they run the tiles of up to 64 rows (measured in
-// grouped_gemm.hpp; at 128 rows the matrix cores and not the loads are the
-// longer part, and the kernels above keep them).
+// kernels take the operands (measured in grouped_gemm.hpp for tiles of up to
+// 64 rows, in grouped_gemm128.hpp for the others).
 template <int NMAT>
 int launch_tiled(hipStream_t s, int quant, GemmArgs a, const PlanView& v, size_t max_rows,
                  bool narrow, bool wave) {
@@ -1159,7 +1186,9 @@ int launch_tiled(hipStream_t s, int quant, GemmArgs a, const PlanView& v, size_t
   if (!narrow) {
     a.tiles = v.l128;
     a.n_tiles = v.counts;
-    if (max_rows > 64 && (st = launch_gemm_q<NMAT, 128>(s, quant, a, unsigned(v.n128)))) return st;
+    if (max_rows > 64 && (st = wave ? launch_tile128_q<NMAT>(s, quant, a, unsigned(v.n128))
+                                    : launch_gemm_q<NMAT, 128>(s, quant, a, unsigned(v.n128))))
+      return st;
     a.tiles = v.l64;
     a.n_tiles = v.counts + 1;
     if (max_rows > 32 && (st = wave ? launch_wave_q<NMAT, 4, 3>(s, quant, a, unsigned(v.n64))

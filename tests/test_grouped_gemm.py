@@ -36,13 +36,31 @@ def _ids(rows, E):
     return np.random.default_rng(3).permutation(ids)
 
 
-def _run(quant, down, H, I, rows, bf16, shift=0):
+D_AT = {Q2_K: (84, 80, 82), Q3_K: (110, 108, None), Q4_K: (144, 0, 2)}  # block, d, dmin
+
+
+def _spread_d(q, mat, seed):
+    """The blocks' d (and dmin) times 2^-8 .. 2^1 each, one in six zero."""
+    nbytes, *at = D_AT[q]
+    b = mat.cpu().numpy().copy().reshape(-1, nbytes)
+    rng = np.random.default_rng(seed)
+    for o in at:
+        if o is not None:
+            d = b[:, o:o + 2].copy().view(np.float16)[:, 0]
+            f = np.exp2(rng.integers(-8, 2, len(d))) * (rng.integers(0, 6, len(d)) > 0)
+            b[:, o:o + 2] = (d * f).astype(np.float16)[:, None].view(np.uint8)
+    return torch.from_numpy(b.reshape(-1)).to(mat.device)
+
+
+def _run(quant, down, H, I, rows, bf16, shift=0, spread=False):
     dev = torch.device("cuda:0")
     E = len(rows)
     ids = _ids(rows, E)
     T = len(ids)
     mats = [ops.synth_quantized(q, 5 + i, 0.02, E * r, c, dev)
             for i, (q, r, c) in enumerate(((quant, I, H), (quant, I, H), (down, H, I)))]
+    if spread:
+        mats = [_spread_d(q, m, 20 + i) for i, (q, m) in enumerate(zip((quant, quant, down), mats))]
     placed = []
     for m in mats:  # the same bytes at an address that is `shift` past an aligned one
         buf = torch.empty(m.numel() + 16, dtype=torch.uint8, device=dev)
@@ -76,6 +94,23 @@ PAIRS = [(Q2_K, Q2_K), (Q3_K, Q3_K), (Q4_K, Q4_K), (Q4_K, Q6_K), (Q2_K, Q3_K)]
                          ids=["to16", "to32", "to64"])
 def test_tile_edges(quant, down, H, I, rows):
     assert _run(quant, down, H, I, rows, bf16=True) < BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,down", PAIRS)
+@pytest.mark.parametrize("H,I", [(512, 512), (768, 256), (256, 768)])
+def test_tile_edges_128(quant, down, H, I):
+    # whole and partial tiles of 128 rows, one expert with two and a remainder
+    assert _run(quant, down, H, I, (65, 127, 128, 129, 0, 275), bf16=True) < BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,down", [(Q2_K, Q2_K), (Q3_K, Q3_K), (Q4_K, Q4_K)])
+@pytest.mark.parametrize("rows", [(128, 100, 0), (64, 32, 16)], ids=["to128", "to64"])
+def test_blocks_of_unlike_or_zero_scale(quant, down, rows):
+    # running sums change their unit from block to block, and a block of d = 0
+    # (or dmin = 0) has none
+    assert _run(quant, down, 1280, 1024, rows, bf16=True, spread=True) < BOUND
 
 
 @pytest.mark.gpu
