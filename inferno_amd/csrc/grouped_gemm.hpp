@@ -71,6 +71,24 @@ struct GemmArgs {
   float* y_out;            // one matrix: fp32 rows [*, N]
 };
 
+// This workgroup's expert and rows [c0, c1) of at most TM; false: none.
+template <int TM>
+__device__ __forceinline__ bool tile_of(const GemmArgs& p, uint32_t& e, uint32_t& c0,
+                                        uint32_t& c1) {
+  if (p.tiles == nullptr) {
+    e = 0;
+    c0 = blockIdx.y * TM;
+    c1 = min(c0 + TM, p.rows);
+  } else {
+    if (blockIdx.y >= *p.n_tiles) return false;
+    const uint4 tile = p.tiles[blockIdx.y];
+    e = tile.x;
+    c0 = tile.y;
+    c1 = tile.z;
+  }
+  return c1 > c0;
+}
+
 __device__ __forceinline__ half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
 __device__ __forceinline__ uint32_t as_u32(half2v v) { return __builtin_bit_cast(uint32_t, v); }
 
@@ -591,10 +609,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 15, g = lane >> 4;
-  if (blockIdx.y >= *p.n_tiles) return;
-  const uint4 tile = p.tiles[blockIdx.y];
-  const uint32_t e = tile.x, c0 = tile.y, c1 = tile.z;
-  if (c1 <= c0) return;
+  uint32_t e, c0, c1;
+  if (!tile_of<TM>(p, e, c0, c1)) return;
   const int n0 = blockIdx.x * TN + wave * RM;  // this wavefront's first row
   const int K = p.K, nkb = K / kUnit;
   uint8_t* const wl = smem_g + wave * WREG;

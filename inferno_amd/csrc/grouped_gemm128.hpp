@@ -203,10 +203,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 31, kg = lane >> 5;
-  if (blockIdx.y >= *p.n_tiles) return;
-  const uint4 tile = p.tiles[blockIdx.y];
-  const uint32_t e = tile.x, c0 = tile.y, c1 = tile.z;
-  if (c1 <= c0) return;
+  uint32_t e, c0, c1;
+  if (!tile_of<128>(p, e, c0, c1)) return;
   const int n0 = blockIdx.x * TN + wave * RM;  // this wavefront's first row
   const int K = p.K, nkb = K / kUnit;
   uint8_t* const wl = smem_g + wave * WREG;

@@ -1222,11 +1222,27 @@ int launch_dense_narrow(hipStream_t s, const GemmArgs& a, unsigned grid_y) {
   return INFERNO_OK;
 }
 
-// Dense GEMMs: tiles of TM rows over all T rows; TM from T so that small
-// batches still spread over the chip (Q8_0 below 128 workgroups of 128-row
-// tiles: 32-row tiles).
+// Dense GEMMs over all T rows. wave: the DMA kernels take the operands, with
+// the widest token tiles that still make enough workgroups; n16 is the number
+// that 16-row tiles would make. Whole layers, shared expert of the staged or
+// fragment-load kernels -> 16- / 32- / 64- / 128-row tiles here: H 2048, Is
+// 768, Q4_K and Q6_K down, T = 64 (n16 48) 110 -> 93 / 99 / 114 / 149 us, T =
+// 512 (384) 242 -> 236 / 233 / 247 / 288, T = 2048 (1536) 590 -> 578 / 555 /
+// 557 / 585, T = 4096 (3072) 1053 -> 1091 / 1045 / 1028 / 1051; H 6144, Is
+// 2048, Q2_K, T = 512 (1024) 1092 -> 1066 / 1052 / 1071 / 1160, T = 4096 (8192)
+// 4140 -> 4404 / 4160 / 4108 / 4030. The others: tiles of TM rows, TM from T
+// so that small batches still spread over the chip (Q8_0 below 128 workgroups
+// of 128-row tiles: 32-row tiles).
 template <int NMAT>
-int launch_dense(hipStream_t s, int quant, GemmArgs a, size_t T) {
+int launch_dense(hipStream_t s, int quant, GemmArgs a, size_t T, bool wave) {
+  if (wave) {
+    auto tiles = [T](size_t rows) { return unsigned((T + rows - 1) / rows); };
+    const size_t n16 = tiles(16) * size_t(a.N / (NMAT == 2 ? 64 : 128));
+    if (n16 <= 256) return launch_wave_q<NMAT, 1, 4>(s, quant, a, tiles(16));
+    if (n16 <= 2048) return launch_wave_q<NMAT, 2, 4>(s, quant, a, tiles(32));
+    if (n16 < 8192) return launch_wave_q<NMAT, 4, 3>(s, quant, a, tiles(64));
+    return launch_tile128_q<NMAT>(s, quant, a, tiles(128));
+  }
   if (T >= 2048) return launch_gemm_q<NMAT, 128>(s, quant, a, unsigned((T + 127) / 128));
   const unsigned gy = unsigned((T + 31) / 32);
   if (quant == INFERNO_Q8_0 && a.N % 32 == 0 && size_t(a.N / 128) * gy < 128 && gemm2_enabled() &&
@@ -1392,8 +1408,7 @@ int launch_prefill_dense(hipStream_t s, int quant, int down_quant, const void* g
   g.N = int(Is);
   g.K = int(H);
   g.h_out = h16;
-  int st;
-  if ((st = launch_dense<2>(s, quant, g, T))) return st;
+  g.in_rows = T;
   GemmArgs d{};
   d.w0 = static_cast<const uint8_t*>(down);
   d.xin = h16;
@@ -1402,7 +1417,12 @@ int launch_prefill_dense(hipStream_t s, int quant, int down_quant, const void* g
   d.N = int(H);
   d.K = int(Is);
   d.y_out = ys;
-  return launch_dense<1>(s, down_quant, d, T);
+  d.in_rows = T;
+  // both or none: the DMA kernels read the group sums that they write
+  const bool wave = quant != INFERNO_Q8_0 && down_quant != INFERNO_Q8_0 &&
+                    wave_gemm_takes(quant, g) && wave_gemm_takes(down_quant, d);
+  if (int st = launch_dense<2>(s, quant, g, T, wave)) return st;
+  return launch_dense<1>(s, down_quant, d, T, wave);
 }
 
 int launch_prefill_combine(hipStream_t s, const float* y, const float* ys, const float* residual,

@@ -190,3 +190,35 @@ def test_layer_decode_and_grouped_agree(quant, shared, T, monkeypatch):
     grouped = layer.forward(x)
     assert float((by_rule - decode).norm() / decode.norm()) < 2e-3
     assert float((grouped - decode).norm() / decode.norm()) < 2e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,down", PAIRS)
+@pytest.mark.parametrize("T,H,Is", [(16, 512, 256), (65, 256, 768), (300, 1024, 2048),
+                                    (1030, 1280, 1024), (2100, 1024, 4096)])
+def test_dense_expert_tiles(quant, down, T, H, Is):
+    # the layer's shared expert over token tiles of 16, 32, 64 and 128 rows
+    # with remainders: what it adds to the same layer without it
+    from inferno_amd import SCORE_SOFTMAX
+    dev = torch.device("cuda:0")
+    E, I, k = 8, 256, 2
+    mats = [ops.synth_quantized(Q4_K, i, 0.02, E * r, c, dev)
+            for i, (r, c) in enumerate(((I, H), (I, H), (H, I)))]
+    sh = [ops.synth_quantized(q, 9 + i, 0.05, r, c, dev)
+          for i, (q, r, c) in enumerate(((quant, Is, H), (quant, Is, H), (down, H, Is)))]
+    g = torch.Generator(device=dev).manual_seed(2)
+    router = torch.randn(E, H, generator=g, device=dev) * 0.02
+    x = torch.randn(T, H, generator=g, device=dev).bfloat16()
+    out = []
+    for shared in (0, Is):
+        kw = dict(shared_gate=sh[0], shared_up=sh[1], shared_down=sh[2], shared_quant=quant,
+                  shared_down_quant=down) if shared else {}
+        layer = ops.MoELayer(
+            hidden=H, experts=E, intermediate=I, top_k=k, quant=Q4_K, down_quant=Q4_K,
+            score_fn=SCORE_SOFTMAX, norm_topk_prob=True, routed_scaling_factor=1.0,
+            router=router, router_bias=None, gate=mats[0], up=mats[1], down=mats[2],
+            shared_intermediate=shared, max_tokens=T, **kw)
+        out.append(layer.forward(x).double())
+    a, b = (x.double() @ ops.dequantize(quant, sh[i]).view(Is, H).double().T for i in (0, 1))
+    ref = (a * torch.sigmoid(a) * b) @ ops.dequantize(down, sh[2]).view(H, Is).double().T
+    assert float((out[1] - out[0] - ref).norm() / ref.norm()) < BOUND
