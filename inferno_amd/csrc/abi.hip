@@ -133,25 +133,22 @@ int run_routed(hipStream_t s, int quant, int down_quant, const void* gate, const
                const MoeScratch& m, bool x_staged, bool mfma, const uint16_t* x16 = nullptr,
                bool distinct_ids = false) {
   int st;
-  // on the MFMA path the dispatch also writes the GEMM's tile lists
-  const PlanOut plan = mfma ? prefill_plan_out(m.plan, T * k, E) : PlanOut{};
-  if ((st = launch_dispatch(s, ids, T, k, E, m.offsets, m.sorted, m.active, mfma ? &plan : nullptr)))
-    return st;
   if (mfma) {
-    if (!x16) {
-      uint16_t* conv = reinterpret_cast<uint16_t*>(m.stage_x);
-      if ((st = launch_to_f16(s, x, x_dtype, T, H, conv))) return st;
-      x16 = conv;
-    }
-    PrefillRouted p{quant, down_quant, gate, up, down, x16, m.offsets, m.sorted, m.active, w,
-                    T, k, E, H, I, reinterpret_cast<uint16_t*>(m.h), m.y, m.plan,
+    uint16_t* const conv = x16 ? nullptr : reinterpret_cast<uint16_t*>(m.stage_x);
+    PrefillRouted p{quant, down_quant, gate, up, down, x16 ? x16 : conv, m.offsets, m.sorted,
+                    m.active, w, T, k, E, H, I, reinterpret_cast<uint16_t*>(m.h), m.y, m.plan,
                     distinct_ids ? T : 0};
+    // the dispatch also writes the GEMM's tile lists
+    const PlanOut plan = prefill_plan_out(p);
+    if ((st = launch_dispatch(s, ids, T, k, E, m.offsets, m.sorted, m.active, &plan))) return st;
+    if (conv && (st = launch_to_f16(s, x, x_dtype, T, H, conv))) return st;
     if ((st = timed(s, kTimerGateUp, "prefill: grouped gate/up GEMMs (gemm_kernel / gemm2_kernel, MFMA)",
                     [&] { return launch_prefill_gate_up(s, p); })))
       return st;
     return timed(s, kTimerDown, "prefill: grouped down GEMMs (gemm_kernel / gemm2_kernel, MFMA)",
                  [&] { return launch_prefill_down(s, p); });
   }
+  if ((st = launch_dispatch(s, ids, T, k, E, m.offsets, m.sorted, m.active, nullptr))) return st;
   // gate/up writes h already staged for the down pass (when the down kind has a
   // packed-f16 kernel; Q6_K reads the fp32 h)
   const bool h_staged = dot2_supported(down_quant);

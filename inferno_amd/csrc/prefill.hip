@@ -869,11 +869,11 @@ __global__ void __launch_bounds__(64 * (SPL ? 2 * WR : WR * WT))
 
 // Upper bounds of the tile lists (grid heights): a 128-row tile covers at
 // least 65 rows, the 64- and 32-row lists hold at most one tile per expert,
-// the 16-row list one per 16 rows when it is the only one.
+// the 16-row list one per 16 rows when it is the only one (narrow).
 size_t bound128(size_t A, size_t E) { return A / 65 + 1; }
 size_t bound_small(size_t A, size_t E) { return std::min(E, A) + 1; }
-size_t bound16(size_t A, size_t E) {
-  return bound_small(A, E) + (prefill_narrow(A, E) ? A / 16 : 0);
+size_t bound16(size_t A, size_t E, bool narrow) {
+  return bound_small(A, E) + (narrow ? A / 16 : 0);
 }
 
 // ----------------------------------------------------------- conversions
@@ -1096,12 +1096,12 @@ struct PlanView {
   size_t n128, n64, n32, n16;
 };
 
-PlanView plan_view(uint32_t* plan, size_t A, size_t E) {
+PlanView plan_view(uint32_t* plan, size_t A, size_t E, bool narrow) {
   PlanView v;
   v.n128 = bound128(A, E);
   v.n64 = bound_small(A, E);
   v.n32 = bound_small(A, E);
-  v.n16 = bound16(A, E);
+  v.n16 = bound16(A, E, narrow);
   v.l128 = reinterpret_cast<uint4*>(plan);
   v.l64 = v.l128 + v.n128;
   v.l32 = v.l64 + v.n64;
@@ -1272,13 +1272,8 @@ bool prefill_dense_supported(int quant, int down_quant, size_t H, size_t Is) {
          Is % kUnit == 0 && H % kTileN == 0 && Is % kTileN == 0;
 }
 
-PlanOut prefill_plan_out(uint32_t* plan, size_t A, size_t E) {
-  const PlanView v = plan_view(plan, A, E);
-  return PlanOut{v.l128, v.l64, v.l32, v.l16, v.counts, prefill_narrow(A, E)};
-}
-
 size_t prefill_plan_words(size_t A, size_t E) {
-  return 4 * (bound128(A, E) + 2 * bound_small(A, E) + bound16(A, E)) + 4;
+  return 4 * (bound128(A, E) + 2 * bound_small(A, E) + bound16(A, E, true)) + 4;
 }
 
 int launch_to_f16(hipStream_t s, const void* x, int x_dtype, size_t rows, size_t K,
@@ -1335,7 +1330,36 @@ GemmArgs down_args(const PrefillRouted& p) {
 bool wave_layer(const PrefillRouted& p) {
   return wave_gemm_takes(p.quant, gate_up_args(p)) && wave_gemm_takes(p.down_quant, down_args(p));
 }
+
+// True when the layer takes 16-row tiles only: one launch per GEMM instead of
+// one per tile size that an expert could fill, and more workgroups; an expert
+// of more rows reads its weights once per 16 (of which L2 and the Infinity
+// Cache hold the later ones).
+// Up to 10 rows per expert on average: 16 caller-routed tokens x 8 over 64
+// experts (2 rows each) 61 -> 52 us, 64 tokens (8 rows) 125 -> 118 us; 32
+// tokens x 10 over 128 experts even; H 6144, I 2048, 256 experts of 8 rows,
+// Q2_K 907 -> 760 us, Q3_K 1060 -> 990, of 11 rows 950 -> 905, 1110 -> 1200.
+// On the DMA kernels also while those tiles make at most 2560 gate/up
+// workgroups (four per CU at a time): whole layers, all tile sizes -> 16-row
+// tiles only: H 2048, I 768, 64 experts, Q4_K, 704 assignments (1296
+// workgroups) 93 -> 68 us, 1536 (1920) 138 -> 91; 16 experts, 2048 (1728) 146
+// -> 92; H 6144, I 2048, 16 experts, 1024 (2560), Q2_K 316 -> 236, Q3_K 372 ->
+// 333, 1536 (3584) 255 -> 311, 290 -> 442; H 4096, I 1536, 32 experts, Q3_K,
+// 1024 (2304) even, 1536 (3072) 175 -> 266.
+constexpr size_t kNarrowRows = 10;
+constexpr size_t kNarrowGroups = 2560;
+bool narrow_layer(const PrefillRouted& p) {
+  const size_t A = p.T * p.k;
+  return A <= kNarrowRows * p.E ||
+         (wave_layer(p) && (p.E + A / 16) * (p.I / 64) <= kNarrowGroups);
+}
 }  // namespace
+
+PlanOut prefill_plan_out(const PrefillRouted& p) {
+  const bool narrow = narrow_layer(p);
+  const PlanView v = plan_view(p.plan, p.T * p.k, p.E, narrow);
+  return PlanOut{v.l128, v.l64, v.l32, v.l16, v.counts, narrow};
+}
 
 int launch_prefill_gate_up(hipStream_t s, const PrefillRouted& p) {
   const size_t A = p.T * p.k;
@@ -1344,15 +1368,17 @@ int launch_prefill_gate_up(hipStream_t s, const PrefillRouted& p) {
     set_error("MFMA prefill path does not cover this layer");
     return INFERNO_ERR_INVALID;
   }
-  return launch_tiled<2>(s, p.quant, gate_up_args(p), plan_view(p.plan, A, p.E),
-                         p.max_rows ? p.max_rows : A, prefill_narrow(A, p.E), wave_layer(p));
+  const bool narrow = narrow_layer(p);
+  return launch_tiled<2>(s, p.quant, gate_up_args(p), plan_view(p.plan, A, p.E, narrow),
+                         p.max_rows ? p.max_rows : A, narrow, wave_layer(p));
 }
 
 int launch_prefill_down(hipStream_t s, const PrefillRouted& p) {
   const size_t A = p.T * p.k;
   if (A == 0) return INFERNO_OK;
-  return launch_tiled<1>(s, p.down_quant, down_args(p), plan_view(p.plan, A, p.E),
-                         p.max_rows ? p.max_rows : A, prefill_narrow(A, p.E), wave_layer(p));
+  const bool narrow = narrow_layer(p);
+  return launch_tiled<1>(s, p.down_quant, down_args(p), plan_view(p.plan, A, p.E, narrow),
+                         p.max_rows ? p.max_rows : A, narrow, wave_layer(p));
 }
 
 // Tokens up to which a layer's Q8_0 shared expert takes the dense Q8_0

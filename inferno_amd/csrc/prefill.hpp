@@ -37,18 +37,6 @@ inline bool grouped_beats_decode(size_t A, size_t H, size_t I, size_t expert_byt
 
 // 32-bit words of the routed planner's scratch (tile lists and counts).
 size_t prefill_plan_words(size_t A, size_t E);
-// The tile lists inside that scratch, for the dispatch launch to fill
-// (launch_dispatch with a plan) before launch_prefill_gate_up reads them.
-PlanOut prefill_plan_out(uint32_t* plan, size_t A, size_t E);
-// True when a batch of A assignments over E experts takes 16-row tiles only.
-// One launch per GEMM instead of one per tile size that an expert could
-// fill; an expert of more rows reads its weights once per 16 (of which L2 and
-// the Infinity Cache hold the later ones). Up to 10 rows per expert on average:
-// 16 caller-routed tokens x 8 over 64 experts (2 rows each) 61 -> 52 us, 64
-// tokens (8 rows) 125 -> 118 us; 32 tokens x 10 over 128 experts even.
-constexpr size_t kNarrowRows = 10;
-inline bool prefill_narrow(size_t A, size_t E) { return A <= kNarrowRows * E; }
-
 // Halfs per row of the f16 activations the grouped GEMMs read (x16, h16): K
 // values, the sums of every 16 of them in two f16 terms (K / 8 halfs: per 256
 // values 16 first terms, then 16 second ones, in the k order of the values),
@@ -90,6 +78,9 @@ struct PrefillRouted {
   size_t max_rows;
 };
 
+// The tile lists of the layer inside p.plan, for the dispatch launch to fill
+// (launch_dispatch with a plan) before launch_prefill_gate_up reads them.
+PlanOut prefill_plan_out(const PrefillRouted& p);
 // Routed gate/up (+SwiGLU, routing weight) over the dispatch groups: plans
 // the expert tiles, then the GEMM; writes h16.
 int launch_prefill_gate_up(hipStream_t s, const PrefillRouted& p);

@@ -12,7 +12,6 @@ import numpy as np
 import pytest
 import torch
 
-import oracle_lib as orc
 from inferno_amd import Q2_K, Q3_K, Q4_K, Q6_K, ops
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -75,10 +74,15 @@ def _run(quant, down, H, I, rows, bf16, shift=0, spread=False):
     again = ops.gguf_moe(*args)
     torch.cuda.synchronize()
     assert torch.equal(out, again)
-    ref = orc.moe_routed(quant, down, *(m.cpu().numpy() for m in mats), x.float().cpu().numpy(),
-                         ids, w.cpu().numpy(), E, 1, I)
-    got = out.cpu().numpy()
-    return float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+    # fp64, expert by expert (the values' own tests compare dequantize with the oracle)
+    deq = [ops.dequantize(q, m).view(E, r, c) for q, m, r, c in
+           ((quant, mats[0], I, H), (quant, mats[1], I, H), (down, mats[2], H, I))]
+    ref = torch.zeros(T, H, dtype=torch.float64, device=dev)
+    for e in range(E):
+        at = torch.from_numpy(np.nonzero(ids == e)[0]).to(dev)
+        gg, uu = (x[at].double() @ d[e].double().T for d in deq[:2])
+        ref[at] = (gg * torch.sigmoid(gg) * uu * w[at, None].double()) @ deq[2][e].double().T
+    return float((out.double() - ref).norm() / ref.norm())
 
 
 # h is rounded to f16 and so are fp32 tokens (2^-12 of a value each, at random);
@@ -87,18 +91,24 @@ BOUND = 2e-3
 PAIRS = [(Q2_K, Q2_K), (Q3_K, Q3_K), (Q4_K, Q4_K), (Q4_K, Q6_K), (Q2_K, Q3_K)]
 
 
+# small layers take 16-row tiles only; these widths (with the rows of MORE, one
+# expert's) the tiles of every size
+WIDE = [(512, 3584), (768, 3840), (256, 3584)]
+MORE = (650,)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("quant,down", PAIRS)
-@pytest.mark.parametrize("H,I", [(512, 512), (768, 256), (256, 768)])
+@pytest.mark.parametrize("H,I", WIDE + [(512, 512), (768, 256), (256, 768)])
 @pytest.mark.parametrize("rows", [(15, 0, 16, 17), (32, 33, 1, 0), (63, 2, 64, 65)],
                          ids=["to16", "to32", "to64"])
 def test_tile_edges(quant, down, H, I, rows):
-    assert _run(quant, down, H, I, rows, bf16=True) < BOUND
+    assert _run(quant, down, H, I, rows + MORE, bf16=True) < BOUND
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("quant,down", PAIRS)
-@pytest.mark.parametrize("H,I", [(512, 512), (768, 256), (256, 768)])
+@pytest.mark.parametrize("H,I", WIDE)
 def test_tile_edges_128(quant, down, H, I):
     # whole and partial tiles of 128 rows, one expert with two and a remainder
     assert _run(quant, down, H, I, (65, 127, 128, 129, 0, 275), bf16=True) < BOUND
@@ -107,10 +117,22 @@ def test_tile_edges_128(quant, down, H, I):
 @pytest.mark.gpu
 @pytest.mark.parametrize("quant,down", [(Q2_K, Q2_K), (Q3_K, Q3_K), (Q4_K, Q4_K)])
 @pytest.mark.parametrize("rows", [(128, 100, 0), (64, 32, 16)], ids=["to128", "to64"])
-def test_blocks_of_unlike_or_zero_scale(quant, down, rows):
+@pytest.mark.parametrize("I", [3584, 1024], ids=["wide", "narrow"])
+def test_blocks_of_unlike_or_zero_scale(quant, down, rows, I):
     # running sums change their unit from block to block, and a block of d = 0
     # (or dmin = 0) has none
-    assert _run(quant, down, 1280, 1024, rows, bf16=True, spread=True) < BOUND
+    assert _run(quant, down, 1280, I, rows + MORE, bf16=True, spread=True) < BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,down", PAIRS)
+@pytest.mark.parametrize("rows", [(160, 0, 1), (31, 17, 200, 48)])
+def test_small_layer_tiles(quant, down, rows):
+    # many 16-row tiles of one expert, against the same rows of weights that
+    # the 16-row rule (like the DMA) leaves to the general kernels
+    a = _run(quant, down, 512, 512, rows, bf16=True)
+    b = _run(quant, down, 512, 512, rows, bf16=True, shift=2)
+    assert a < BOUND and b < BOUND and a <= 1.05 * b
 
 
 @pytest.mark.gpu
@@ -195,7 +217,8 @@ def test_layer_decode_and_grouped_agree(quant, shared, T, monkeypatch):
 @pytest.mark.gpu
 @pytest.mark.parametrize("quant,down", PAIRS)
 @pytest.mark.parametrize("T,H,Is", [(16, 512, 256), (65, 256, 768), (300, 1024, 2048),
-                                    (1030, 1280, 1024), (2100, 1024, 4096)])
+                                    (1030, 1280, 1024), (2100, 1280, 1536),
+                                    (2100, 1024, 4096)])
 def test_dense_expert_tiles(quant, down, T, H, Is):
     # the layer's shared expert over token tiles of 16, 32, 64 and 128 rows
     # with remainders: what it adds to the same layer without it
