@@ -633,8 +633,11 @@ bool layer_takes_decode(const inferno_moe_layer* L, size_t T, int x_dtype) {
   if (T == 1) return true;
   const size_t H = L->hidden, I = L->intermediate, k = L->top_k;
   if (use_mfma(L->quant, L->down_quant, T, k, L->experts, H, I, Is)) return false;
-  // (a threshold given in the environment is the only rule then)
-  return std::getenv("INFERNO_PREFILL_MIN_ASSIGNMENTS") != nullptr ||
+  // (a threshold given in the environment is the only rule then; weights that
+  // the LDS DMA cannot take stay here, the general GEMMs were not weighed)
+  const uintptr_t at = reinterpret_cast<uintptr_t>(L->gate) | reinterpret_cast<uintptr_t>(L->up) |
+                       reinterpret_cast<uintptr_t>(L->down);
+  return std::getenv("INFERNO_PREFILL_MIN_ASSIGNMENTS") != nullptr || at % 16 != 0 ||
          !prefill_routed_supported(L->quant, L->down_quant, H, I, L->experts) ||
          !grouped_beats_decode(T * k, H, I,
                                2 * matrix_bytes(L->quant, I, H) + matrix_bytes(L->down_quant, H, I),
