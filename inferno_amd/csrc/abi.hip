@@ -633,6 +633,9 @@ bool layer_takes_decode(const inferno_moe_layer* L, size_t T, int x_dtype) {
   if (T == 1) return true;
   const size_t H = L->hidden, I = L->intermediate, k = L->top_k;
   if (use_mfma(L->quant, L->down_quant, T, k, L->experts, H, I, Is)) return false;
+  // fp32 tokens enter the decode launches as two f16 terms (22 bits), the
+  // grouped GEMMs as one
+  if (x_dtype != INFERNO_BF16) return true;
   // (a threshold given in the environment is the only rule then; weights that
   // the LDS DMA cannot take stay here, the general GEMMs were not weighed)
   const uintptr_t at = reinterpret_cast<uintptr_t>(L->gate) | reinterpret_cast<uintptr_t>(L->up) |
@@ -656,7 +659,8 @@ bool layer_takes_grouped(const inferno_moe_layer* L, size_t T, int x_dtype) {
   const bool shared_q8 = Is == 0 || (sq == INFERNO_Q8_0 && sdq == INFERNO_Q8_0);
   if (use_mfma(L->quant, L->down_quant, T, L->top_k, L->experts, L->hidden, L->intermediate, Is))
     return true;
-  return shared_q8 && T > 1 && std::getenv("INFERNO_PREFILL_MIN_ASSIGNMENTS") == nullptr &&
+  return shared_q8 && T > 1 && x_dtype == INFERNO_BF16 &&
+         std::getenv("INFERNO_PREFILL_MIN_ASSIGNMENTS") == nullptr &&
          prefill_routed_supported(L->quant, L->down_quant, L->hidden, L->intermediate, L->experts) &&
          decode_supported(T, L->top_k, L->experts, L->hidden, L->intermediate, Is, x_dtype,
                           L->quant, L->down_quant);
