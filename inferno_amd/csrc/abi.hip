@@ -387,7 +387,7 @@ int inferno_q8_0_gate_up_swiglu(void* stream, const void* gate, size_t gate_byte
     p.x = static_cast<uint16_t*>(workspace);
     p.terms = x_dtype == INFERNO_BF16 ? 1 : 2;
     p.pitch = dense_q8_pitch(H, p.terms);
-    p.scaled = true;
+    p.scale_at = size_t(p.terms) * H;
     p.T = T;
     p.K = H;
     p.N = Is;
@@ -421,7 +421,7 @@ int inferno_q8_0_matvec_add2(void* stream, const void* w, size_t w_bytes, const 
     p.x = static_cast<uint16_t*>(workspace);
     p.terms = 2;
     p.pitch = dense_q8_pitch(In, 2);
-    p.scaled = true;
+    p.scale_at = 2 * In;
     p.T = T;
     p.K = In;
     p.N = O;

@@ -12,17 +12,23 @@
 // and moved to registers whole before the next unit's copies go out. No
 // barrier until the sums of the wavefronts are added, in their order.
 //
-// Measured, H 6144 and Is 2048, both entry points together (stage, gate/up,
-// stage, down), against the packed-f16 GEMVs they replace: 16 tokens 127 ->
-// 28 us (gate/up 8 us for 27 MB), 1 token 27 -> 26, 4 42 -> 26, 512 1540 ->
-// 427; error against fp64 1.5e-6 -> 1.6e-7.
+// Measured, H 6144 and Is 2048, bf16 tokens, both entry points together (stage,
+// gate/up, stage, down), against the packed-f16 GEMVs they replace: 16 tokens
+// 127 -> 26 us, 4 40 -> 28, 1 even, 128 938 -> 116, 512 3700 -> 435; error
+// against fp64 of the gate/up 2.4e-7 -> 1.6e-7 (fp32 tokens 1.3e-6 -> 2.2e-7),
+// of the down 2.2e-6 -> 1.3e-7. The scales cost 8 % of the gate/up at 512
+// tokens (172 us without) and nothing of the down.
 //
 // The codes enter the MFMA as exact f16 integers, each 32-value block's sums
 // are scaled by its d in fp32. Tokens are one f16 term (bf16 values, or the
 // layer's f16 rows) or two (fp32 values: 22 bits), in units of a power of two
-// per row that puts the row's largest value at 2^14 .. 2^15, so that what f16
-// cannot hold of a row lies 2^-39 below its largest value.
+// that puts the largest value of each 32 (a weight block's own width) at 2^14
+// .. 2^15: what f16 cannot hold of a value lies 2^-39 below the largest one of
+// its block, whatever the rest of the row holds. A unit for the whole row
+// instead loses a row beside one large value.
 #include "dense_q8.hpp"
+
+#include <cfloat>
 
 #include "gemv_common.hpp"
 
@@ -45,45 +51,54 @@ __device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint8_t
 
 // ------------------------------------------------------------------- staging
 
-// One row per workgroup: the power of two that puts the largest value in
-// [2^14, 2^15), then the terms.
+// A wavefront per 256 values of a row, four to a lane; eight lanes share the
+// power of two of their 32 values.
 template <typename XT, int TERMS>
 __global__ void __launch_bounds__(256)
     stage_kernel(const XT* __restrict__ x, int K, uint16_t* __restrict__ staged) {
-  __shared__ float wmax[4];
-  const int tid = threadIdx.x;
-  const XT* row = x + size_t(blockIdx.x) * K;
+  const int lane = threadIdx.x & 63, kb = int(blockIdx.y) * 4 + int(threadIdx.x >> 6);
+  if (kb * kUnit >= K) return;
+  const int at = kb * kUnit + 4 * lane;
+  const uint8_t* src = reinterpret_cast<const uint8_t*>(x + size_t(blockIdx.x) * K + at);
   uint16_t* out = staged + size_t(blockIdx.x) * dense_q8_pitch(K, TERMS);
-  float m = 0.f;
-  for (int c = tid; c < K / 8; c += 256)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float v = fabsf(to_f32(row[8 * c + j]));
-      m = v < 3.0e38f ? fmaxf(m, v) : m;  // infinities and NaN keep their own rows only
-    }
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, kWave));
-  if ((tid & 63) == 0) wmax[tid >> 6] = m;
-  __syncthreads();
-  m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-  const int e = m > 0.f ? 14 - int((f32_to_bits(m) >> 23) & 255u) + 127 : 0;
-  // (a subnormal m has exponent field 0: e = 141 puts it below 2^15 all the same)
-  if (tid == 0) *reinterpret_cast<float*>(out + size_t(TERMS) * K) = __builtin_amdgcn_ldexpf(1.f, -e);
-  for (int c = tid; c < K / 8; c += 256) {
-    _Float16 hi[8], lo[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float v = __builtin_amdgcn_ldexpf(to_f32(row[8 * c + j]), e);
-      hi[j] = (_Float16)v;
-      lo[j] = (_Float16)(v - (float)hi[j]);
-    }
-    auto put = [&](uint16_t* o, const _Float16* v) {  // k order 0 2 1 3 4 6 5 7
-      const half8 r = {v[0], v[2], v[1], v[3], v[4], v[6], v[5], v[7]};
-      *reinterpret_cast<half8*>(o + 8 * c) = r;
-    };
-    put(out, hi);
-    if constexpr (TERMS == 2) put(out + K, lo);
+  float v[4];
+  if constexpr (sizeof(XT) == 2) {
+    const uint2 w = ld_u2(src);
+    v[0] = bits_to_f32(w.x << 16);
+    v[1] = bits_to_f32(w.x & 0xffff0000u);
+    v[2] = bits_to_f32(w.y << 16);
+    v[3] = bits_to_f32(w.y & 0xffff0000u);
+  } else {
+    const uint4 w = ld_u4(src);
+    v[0] = bits_to_f32(w.x);
+    v[1] = bits_to_f32(w.y);
+    v[2] = bits_to_f32(w.z);
+    v[3] = bits_to_f32(w.w);
   }
+  float m = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) m = fabsf(v[j]) <= FLT_MAX ? fmaxf(m, fabsf(v[j])) : m;
+#pragma unroll
+  for (int o = 1; o < 8; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, kWave));
+  const int e = m > 0.f ? 141 - int((f32_to_bits(m) >> 23) & 255u) : 0;
+  // (a subnormal m has exponent field 0: e = 141 puts it below 2^15 all the same)
+  if ((lane & 7) == 0)
+    reinterpret_cast<float*>(out + size_t(TERMS) * K)[kb * 8 + lane / 8] =
+        __builtin_amdgcn_ldexpf(1.f, -e);
+  _Float16 hi[4], lo[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float u = __builtin_amdgcn_ldexpf(v[j], e);
+    hi[j] = (_Float16)u;
+    lo[j] = (_Float16)(u - (float)hi[j]);
+  }
+  auto put = [&](uint16_t* o, const _Float16* q) {  // k order 0 2 1 3 within four
+    const half2v a = {q[0], q[2]}, b = {q[1], q[3]};
+    *reinterpret_cast<uint2*>(o + at) =
+        make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
+  };
+  put(out, hi);
+  if constexpr (TERMS == 2) put(out + K, lo);
 }
 
 // ---------------------------------------------------------------------- GEMM
@@ -103,19 +118,22 @@ __device__ __forceinline__ half8 codes8(uint32_t w0, uint32_t w1) {
                                               pair(b, 0x04020400u), pair(b, 0x04030401u)));
 }
 
-template <int NB, int TERMS, int WAVES>
+// A wavefront's region: weights, tokens, the scales of 16 rows x 8 blocks.
+template <int NB, int TERMS, int WAVES, bool SCALED>
 constexpr size_t lds_bytes() {
-  const size_t wave = kRows * kUnitBytes + size_t(NB) * TERMS * 16 * kUnit * 2;
+  const size_t wave =
+      kRows * kUnitBytes + size_t(NB) * TERMS * 16 * kUnit * 2 + (SCALED ? size_t(NB) * 512 : 0);
   return WAVES * wave;  // the sums passed between wavefronts take less
 }
 
 // NMAT = 2: gate rows n0 .. + 7 are the workgroup's rows 0 .. 7, up rows
 // n0 .. + 7 its rows 8 .. 15; NMAT = 1: rows n0 .. + 15.
-template <int NMAT, int NB, int TERMS, int WAVES>
+template <int NMAT, int NB, int TERMS, int WAVES, bool SCALED>
 __global__ void __launch_bounds__(64 * WAVES) dense_q8_kernel(DenseQ8 p) {
   constexpr int TM = 16 * NB, TN = kRows / NMAT;
   constexpr int WBYTES = kRows * kUnitBytes, XBYTES = NB * TERMS * 16 * kUnit * 2;
-  static_assert(WAVES * NB * 4 * 64 * 4 <= int(lds_bytes<NB, TERMS, WAVES>()), "sums fit");
+  constexpr int SBYTES = SCALED ? NB * 512 : 0;
+  static_assert(WAVES * NB * 4 * 64 * 4 <= int(lds_bytes<NB, TERMS, WAVES, SCALED>()), "sums fit");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_d[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -124,8 +142,9 @@ __global__ void __launch_bounds__(64 * WAVES) dense_q8_kernel(DenseQ8 p) {
   const int n0 = blockIdx.x * TN, t0 = blockIdx.y * TM;
   const int nkb = K / kUnit;
   const uint32_t row_bytes = uint32_t(nkb) * kUnitBytes;
-  uint8_t* const wl = smem_d + wave * (WBYTES + XBYTES);
+  uint8_t* const wl = smem_d + wave * (WBYTES + XBYTES + SBYTES);
   uint8_t* const xl = wl + WBYTES;
+  uint8_t* const sl = xl + XBYTES;
 
   // weight DMA: 17 lanes per row, three rows per instruction; rows past the
   // matrix are copies of its last one (not stored)
@@ -163,6 +182,12 @@ __global__ void __launch_bounds__(64 * WAVES) dense_q8_kernel(DenseQ8 p) {
                   uint32_t(r) * xpitch + 16 * ((lane & 31) ^ (r & 15)),
                   xl + ((nb * TERMS + t) * 16 + 2 * u) * 512);
         }
+    if constexpr (SCALED)  // the unit's eight scales of a row are two pieces
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        if (lane < 32 && t0 + 16 * nb + (lane >> 1) < T)
+          dma16(xin + p.scale_at * 2 + size_t(kb) * 32,
+                uint32_t(16 * nb + (lane >> 1)) * xpitch + 16 * (lane & 1), sl + nb * 512);
   };
 
   floatx4 acc[NB];
@@ -174,6 +199,7 @@ __global__ void __launch_bounds__(64 * WAVES) dense_q8_kernel(DenseQ8 p) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's own copies
     uint32_t ev[4][3], od[4][2], ds[4];
     half8 x[NB][TERMS][8];
+    floatx4 sc[SCALED ? NB : 1][4][2];  // of token 4 g + v: blocks 0 .. 3, 4 .. 7
 #pragma unroll
     for (int c = 0; c < 4; ++c) {  // blocks 2 c and 2 c + 1
 #pragma unroll
@@ -190,6 +216,14 @@ __global__ void __launch_bounds__(64 * WAVES) dense_q8_kernel(DenseQ8 p) {
         for (int k = 0; k < 8; ++k)
           x[nb][t][k] = *reinterpret_cast<const half8*>(xl + ((nb * TERMS + t) * 16 + i) * 512 +
                                                         16 * ((4 * k + g) ^ i));
+    if constexpr (SCALED)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            sc[nb][v][j] = *reinterpret_cast<const floatx4*>(sl + (16 * nb + 4 * g + v) * 32 + 16 * j);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (kb + WAVES < nkb) issue(kb + WAVES);
 #pragma unroll
@@ -205,7 +239,9 @@ __global__ void __launch_bounds__(64 * WAVES) dense_q8_kernel(DenseQ8 p) {
 #pragma unroll
         for (int t = TERMS - 1; t >= 0; --t)
           part = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[nb][t][k], w, part, 0, 0, 0);
-        acc[nb] += part * d;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)  // (the scale, a power of two, rounds nothing)
+          acc[nb][v] += (SCALED ? part[v] * sc[nb][v][k >> 2][k & 3] : part[v]) * d;
       }
     }
   }
@@ -224,9 +260,7 @@ __global__ void __launch_bounds__(64 * WAVES) dense_q8_kernel(DenseQ8 p) {
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int t = t0 + 16 * wave + 4 * g + v;
-    float y = s[v];
-    if (p.scaled && t < T)
-      y *= *reinterpret_cast<const float*>(p.x + size_t(t) * p.pitch + size_t(TERMS) * K);
+    const float y = s[v];
     if constexpr (NMAT == 2) {
       const float up = __shfl_xor(y, 8, 16);
       const int n = n0 + i;
@@ -249,10 +283,10 @@ __global__ void __launch_bounds__(64 * WAVES) dense_q8_kernel(DenseQ8 p) {
   }
 }
 
-template <int NMAT, int NB, int TERMS, int WAVES>
+template <int NMAT, int NB, int TERMS, int WAVES, bool SCALED>
 int launch(hipStream_t s, const DenseQ8& p) {
-  constexpr size_t lds = lds_bytes<NB, TERMS, WAVES>();
-  auto kern = dense_q8_kernel<NMAT, NB, TERMS, WAVES>;
+  constexpr size_t lds = lds_bytes<NB, TERMS, WAVES, SCALED>();
+  auto kern = dense_q8_kernel<NMAT, NB, TERMS, WAVES, SCALED>;
   if constexpr (lds > 64 * 1024) {
     static const hipError_t attr = hipFuncSetAttribute(
         reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
@@ -265,15 +299,24 @@ int launch(hipStream_t s, const DenseQ8& p) {
   return INFERNO_OK;
 }
 
-template <int NMAT, int NB, int TERMS>
+template <int NMAT, int NB, int TERMS, bool SCALED>
 int launch_waves(hipStream_t s, const DenseQ8& p) {
   // few workgroups and a long K: as many wavefronts split it as LDS takes (up
   // to eight), so that a CU with one workgroup has more in flight
   constexpr int kMany = NB * TERMS == 1 ? 8 : 6;
-  static_assert(lds_bytes<NB, TERMS, kMany>() <= 160 * 1024, "LDS of a CU");
+  static_assert(lds_bytes<NB, TERMS, kMany, SCALED>() <= 160 * 1024, "LDS of a CU");
   const size_t wgs = (p.N * NMAT + kRows - 1) / kRows * ((p.T + 16 * NB - 1) / (16 * NB));
-  if (wgs <= 384 && p.K / kUnit >= 16) return launch<NMAT, NB, TERMS, kMany>(s, p);
-  return launch<NMAT, NB, TERMS, 4>(s, p);
+  if (wgs <= 384 && p.K / kUnit >= 16) return launch<NMAT, NB, TERMS, kMany, SCALED>(s, p);
+  return launch<NMAT, NB, TERMS, 4, SCALED>(s, p);
+}
+
+// 32 tokens per workgroup only with one term (two would take 128 registers).
+template <int NMAT>
+int launch_terms(hipStream_t s, const DenseQ8& p) {
+  if (p.terms == 2) return launch_waves<NMAT, 1, 2, true>(s, p);
+  if (p.scale_at)
+    return p.T > 16 ? launch_waves<NMAT, 2, 1, true>(s, p) : launch_waves<NMAT, 1, 1, true>(s, p);
+  return p.T > 16 ? launch_waves<NMAT, 2, 1, false>(s, p) : launch_waves<NMAT, 1, 1, false>(s, p);
 }
 
 }  // namespace
@@ -286,28 +329,22 @@ bool dense_q8_takes(size_t T, const void* w0, const void* w1, const void* rows) 
 
 int launch_dense_q8_stage(hipStream_t s, const void* x, int x_dtype, size_t T, size_t K,
                           uint16_t* staged) {
+  const dim3 grid{unsigned(T), unsigned((K / kUnit + 3) / 4)};
   if (x_dtype == INFERNO_BF16)
-    stage_kernel<uint16_t, 1><<<unsigned(T), 256, 0, s>>>(static_cast<const uint16_t*>(x), int(K), staged);
+    stage_kernel<uint16_t, 1><<<grid, 256, 0, s>>>(static_cast<const uint16_t*>(x), int(K), staged);
   else
-    stage_kernel<float, 2><<<unsigned(T), 256, 0, s>>>(static_cast<const float*>(x), int(K), staged);
+    stage_kernel<float, 2><<<grid, 256, 0, s>>>(static_cast<const float*>(x), int(K), staged);
   INF_LAUNCHED();
   return INFERNO_OK;
 }
 
 int launch_dense_q8(hipStream_t s, const DenseQ8& p) {
   if (p.T == 0) return INFERNO_OK;
-  if (p.K % kUnit || p.N == 0 || !(p.terms == 1 || p.terms == 2)) {
-    set_error("dense Q8_0 GEMM: K must be a multiple of 256, one or two terms");
+  if (p.K % kUnit || p.N == 0 || !(p.terms == 1 || (p.terms == 2 && p.scale_at))) {
+    set_error("dense Q8_0 GEMM: K must be a multiple of 256, one term or two scaled ones");
     return INFERNO_ERR_INVALID;
   }
-  // 32 tokens per workgroup only with one term (two would take 128 registers)
-  const bool wide = p.T > 16 && p.terms == 1;
-  if (p.w1) {
-    if (p.terms == 2) return launch_waves<2, 1, 2>(s, p);
-    return wide ? launch_waves<2, 2, 1>(s, p) : launch_waves<2, 1, 1>(s, p);
-  }
-  if (p.terms == 2) return launch_waves<1, 1, 2>(s, p);
-  return wide ? launch_waves<1, 2, 1>(s, p) : launch_waves<1, 1, 1>(s, p);
+  return p.w1 ? launch_terms<2>(s, p) : launch_terms<1>(s, p);
 }
 
 }  // namespace inferno

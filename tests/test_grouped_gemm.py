@@ -183,6 +183,36 @@ def test_dense_q8_rows(T, H, Is, bf16):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 16, 40])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_dense_q8_rows_beside_a_large_value(T, bf16):
+    # one activation of 1e10 per row that meets weight blocks of d = 0: what it
+    # takes from f16's range is its own 32 values', not the row's (1e-5 as above)
+    dev = torch.device("cuda:0")
+    from inferno_amd import Q8_0
+    H, Is, at = 1024, 200, 330
+    g = torch.Generator(device=dev).manual_seed(11)
+    x = torch.randn(T, H, generator=g, device=dev)
+    x[:, at] = 1e10
+    x = x.bfloat16() if bf16 else x
+
+    def weights(seed, rows):
+        w = ops.synth_quantized(Q8_0, seed, 0.02, rows, H, dev).view(rows, H // 32, 34).clone()
+        w[:, at // 32, :2] = 0
+        return w.view(-1)
+
+    wg, wu, wd = (weights(s, Is) for s in (1, 2, 3))
+    a, b, c = (x.double() @ ops.dequantize(Q8_0, w).view(Is, H).double().T for w in (wg, wu, wd))
+    ref = a * torch.sigmoid(a) * b
+    h = ops.q8_0_gate_up_swiglu(wg, wu, x, Is)
+    assert float((h - ref).norm() / ref.norm()) < 1e-5
+    ra = torch.randn(T, Is, generator=g, device=dev)
+    if not bf16:  # (the matvec takes fp32 rows)
+        out = ops.q8_0_matvec_add2(wd, x, ra, None, Is)
+        assert float((out - ra - c).norm() / c.norm()) < 1e-5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [2, 3, 4, 6])
 @pytest.mark.parametrize("shared", [0, 1024])
 @pytest.mark.parametrize("quant", [Q2_K, Q3_K, Q4_K])
