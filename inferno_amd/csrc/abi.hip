@@ -137,7 +137,7 @@ int run_routed(hipStream_t s, int quant, int down_quant, const void* gate, const
     uint16_t* const conv = x16 ? nullptr : reinterpret_cast<uint16_t*>(m.stage_x);
     PrefillRouted p{quant, down_quant, gate, up, down, x16 ? x16 : conv, m.offsets, m.sorted,
                     m.active, w, T, k, E, H, I, reinterpret_cast<uint16_t*>(m.h), m.y, m.plan,
-                    distinct_ids ? T : 0};
+                    distinct_ids ? T : 0, nullptr};
     // the dispatch also writes the GEMM's tile lists
     const PlanOut plan = prefill_plan_out(p);
     if ((st = launch_dispatch(s, ids, T, k, E, m.offsets, m.sorted, m.active, &plan))) return st;
@@ -619,51 +619,98 @@ bool layer_shared_slot(const inferno_moe_layer* L, size_t T, int x_dtype) {
                                       x_dtype, L->quant, L->down_quant);
 }
 
-// True when the layer forward takes the fused decode launches for T tokens.
-bool layer_takes_decode(const inferno_moe_layer* L, size_t T, int x_dtype) {
-  const size_t Is = L->shared_intermediate;
-  const int sq = L->shared_quant ? L->shared_quant : INFERNO_Q8_0;
-  const int sdq = L->shared_down_quant ? L->shared_down_quant : INFERNO_Q8_0;
-  const bool shared_q8 = Is == 0 || (sq == INFERNO_Q8_0 && sdq == INFERNO_Q8_0);
-  if (layer_shared_slot(L, T, x_dtype)) return true;
-  if (!decode_supported(T, L->top_k, L->experts, L->hidden, L->intermediate, Is, x_dtype,
-                        L->quant, L->down_quant) ||
-      !shared_q8)
+// How the layer forward runs T tokens.
+enum class LayerPath {
+  kDecode,   // the fused decode launches
+  kFew,      // a few tokens on the grouped GEMMs, scaled rows
+  kGrouped,  // the grouped GEMMs
+  kStages,   // the stage-by-stage GEMVs
+};
+
+// True when a layer of several tokens that the decode launches take runs on
+// the grouped GEMMs instead: bf16 tokens (fp32 ones enter the decode launches
+// as two f16 terms, the GEMMs as one), every matrix and the workspace where
+// the LDS DMA can copy them, and bytes that outweigh the launches.
+// INFERNO_DECODE_GROUPED: 0 never, 1 wherever the kernels take the layer; a
+// threshold of assignments given in the environment is the only rule else.
+bool layer_takes_few(const inferno_moe_layer* L, size_t T, int x_dtype, const void* workspace) {
+  const size_t H = L->hidden, I = L->intermediate, Is = L->shared_intermediate;
+  if (x_dtype != INFERNO_BF16 || switch_off("INFERNO_DECODE_GROUPED") ||
+      !prefill_few_takes(L->quant, L->down_quant, L->gate, L->up, L->down, workspace, H, I,
+                         L->experts) ||
+      (Is && !(dense_q8_takes(T, L->shared_gate, L->shared_up, workspace) &&
+               dense_q8_takes(T, L->shared_down, nullptr, workspace))))
     return false;
-  if (T == 1) return true;
-  const size_t H = L->hidden, I = L->intermediate, k = L->top_k;
-  if (use_mfma(L->quant, L->down_quant, T, k, L->experts, H, I, Is)) return false;
-  // fp32 tokens enter the decode launches as two f16 terms (22 bits), the
-  // grouped GEMMs as one
-  if (x_dtype != INFERNO_BF16) return true;
-  // (a threshold given in the environment is the only rule then; weights that
-  // the LDS DMA cannot take stay here, the general GEMMs were not weighed)
-  const uintptr_t at = reinterpret_cast<uintptr_t>(L->gate) | reinterpret_cast<uintptr_t>(L->up) |
-                       reinterpret_cast<uintptr_t>(L->down);
-  return std::getenv("INFERNO_PREFILL_MIN_ASSIGNMENTS") != nullptr || at % 16 != 0 ||
-         !prefill_routed_supported(L->quant, L->down_quant, H, I, L->experts) ||
-         !grouped_beats_decode(T * k, H, I,
-                               2 * matrix_bytes(L->quant, I, H) + matrix_bytes(L->down_quant, H, I),
-                               Is != 0);
+  if (switch_on("INFERNO_DECODE_GROUPED")) return true;
+  return std::getenv("INFERNO_PREFILL_MIN_ASSIGNMENTS") == nullptr &&
+         grouped_beats_decode(T * L->top_k, 2 * matrix_bytes(L->quant, I, H) +
+                                                matrix_bytes(L->down_quant, H, I));
 }
 
-// True when a layer forward that does not take the decode launches runs its
-// routed experts on the grouped GEMMs: those of decode_supported shapes
-// always do (layer_takes_decode has weighed the two), others from the
-// assignment counts of use_mfma (below them their GEMV kernels keep fp32
-// activations).
-bool layer_takes_grouped(const inferno_moe_layer* L, size_t T, int x_dtype) {
+LayerPath layer_path(const inferno_moe_layer* L, size_t T, int x_dtype, const void* workspace) {
   const size_t Is = L->shared_intermediate;
   const int sq = L->shared_quant ? L->shared_quant : INFERNO_Q8_0;
   const int sdq = L->shared_down_quant ? L->shared_down_quant : INFERNO_Q8_0;
-  const bool shared_q8 = Is == 0 || (sq == INFERNO_Q8_0 && sdq == INFERNO_Q8_0);
+  if (layer_shared_slot(L, T, x_dtype)) return LayerPath::kDecode;
+  const bool decode = (Is == 0 || (sq == INFERNO_Q8_0 && sdq == INFERNO_Q8_0)) &&
+                      decode_supported(T, L->top_k, L->experts, L->hidden, L->intermediate, Is,
+                                       x_dtype, L->quant, L->down_quant);
+  if (decode && T == 1) return LayerPath::kDecode;
+  // from these counts the grouped GEMMs read each expert's weights once for
+  // all its tokens
   if (use_mfma(L->quant, L->down_quant, T, L->top_k, L->experts, L->hidden, L->intermediate, Is))
-    return true;
-  return shared_q8 && T > 1 && x_dtype == INFERNO_BF16 &&
-         std::getenv("INFERNO_PREFILL_MIN_ASSIGNMENTS") == nullptr &&
-         prefill_routed_supported(L->quant, L->down_quant, L->hidden, L->intermediate, L->experts) &&
-         decode_supported(T, L->top_k, L->experts, L->hidden, L->intermediate, Is, x_dtype,
-                          L->quant, L->down_quant);
+    return LayerPath::kGrouped;
+  if (!decode) return LayerPath::kStages;
+  return layer_takes_few(L, T, x_dtype, workspace) ? LayerPath::kFew : LayerPath::kDecode;
+}
+
+// A few tokens after their router: the grouped GEMMs over rows of x and h that
+// are scaled by themselves, since the decode launches (the other path of the
+// same calls) take activations of any size. x and h pass through a launch that
+// scales them, h (the routed rows and the shared expert's in one) from fp32.
+int layer_few(hipStream_t s, const inferno_moe_layer* L, const void* x, int x_dtype,
+              const float* residual, size_t T, float* out, const uint32_t* ids, const float* wts,
+              const LayerScratch& w) {
+  const size_t H = L->hidden, E = L->experts, I = L->intermediate, k = L->top_k, A = T * k;
+  const size_t Is = L->shared_intermediate;
+  uint16_t* const x16 = reinterpret_cast<uint16_t*>(w.moe.stage_x);
+  uint16_t* const h16 = reinterpret_cast<uint16_t*>(w.moe.stage_h);
+  uint16_t* const hs16 = reinterpret_cast<uint16_t*>(w.stage_hs);
+  PrefillRouted p{L->quant, L->down_quant, L->gate, L->up, L->down, x16, w.moe.offsets,
+                  w.moe.sorted, w.moe.active, wts, T, k, E, H, I, h16, w.moe.y, w.moe.plan, T,
+                  w.moe.h};
+  DenseQ8 g{}, d{};  // the shared expert
+  g.terms = d.terms = 1;
+  g.T = d.T = T;
+  g.w0 = L->shared_gate;
+  g.w1 = L->shared_up;
+  g.x = x16;
+  g.pitch = f16_scaled_pitch(H);
+  g.scale_at = f16_scale_at(H);
+  g.K = d.N = H;
+  g.N = d.K = Is;
+  g.out = w.hs;
+  d.w0 = L->shared_down;
+  d.x = hs16;
+  d.pitch = f16_scaled_pitch(Is);
+  d.scale_at = f16_scale_at(Is);
+  d.out = w.ys;
+  const PlanOut plan = prefill_plan_out(p);
+  int st;
+  if ((st = launch_dispatch(s, ids, T, k, E, w.moe.offsets, w.moe.sorted, w.moe.active, &plan)))
+    return st;
+  if ((st = launch_scaled_rows(s, x_dtype, {x, x16, T, H}, {}))) return st;
+  if ((st = timed(s, kTimerGateUp, "grouped, few tokens: gate/up GEMM (wave_gemm_kernel, scaled rows)",
+                  [&] { return launch_prefill_gate_up(s, p); })))
+    return st;
+  if (Is && (st = launch_dense_q8(s, g))) return st;
+  if ((st = launch_scaled_rows(s, INFERNO_F32, {w.moe.h, h16, A, I}, {w.hs, hs16, Is ? T : 0, Is})))
+    return st;
+  if ((st = timed(s, kTimerDown, "grouped, few tokens: down GEMM (wave_gemm_kernel, scaled rows)",
+                  [&] { return launch_prefill_down(s, p); })))
+    return st;
+  if (Is && (st = launch_dense_q8(s, d))) return st;
+  return launch_prefill_combine(s, w.moe.y, Is ? w.ys : nullptr, residual, T, k, H, out);
 }
 
 // logits_ready: the tokens' router logits [T, E], already formed (the
@@ -715,10 +762,8 @@ int layer_forward(void* stream, const inferno_moe_layer* L, const void* x, int x
   hipStream_t s = as_stream(stream);
   uint32_t* ids = expert_ids_out ? expert_ids_out : w.ids;
   float* wts = expert_weights_out ? expert_weights_out : w.weights;
-  // the fused decode path below the grouped GEMM's assignment threshold
-  // (use_mfma; and for one token); from there the grouped MFMA GEMM reads
-  // each expert's weights once for all its tokens
-  const bool decode = layer_takes_decode(L, T, x_dtype);
+  const LayerPath path = layer_path(L, T, x_dtype, workspace);
+  const bool decode = path == LayerPath::kDecode;
   if (logits_ready && !decode) {
     set_error("precomputed logits need the decode path");
     return INFERNO_ERR_INVALID;
@@ -754,7 +799,7 @@ int layer_forward(void* stream, const inferno_moe_layer* L, const void* x, int x
   const bool router_blas = w.rblas != nullptr && w.blas_lib != nullptr &&
                            router_blas_takes(T, H, E, x_dtype);
   const int parts = router_blas ? 1 : router_logit_parts(T, H, E, x_dtype);
-  const bool mfma_path = layer_takes_grouped(L, T, x_dtype);
+  const bool mfma_path = path == LayerPath::kGrouped;
   // the shared expert on the dense MFMA GEMMs when its formats have them
   // (Q8_0; the Laguna XS Q4_K gate/up with Q4_K or Q6_K down), else on the
   // GEMV kernels
@@ -778,6 +823,8 @@ int layer_forward(void* stream, const inferno_moe_layer* L, const void* x, int x
                                L->norm_topk_prob, L->routed_scaling_factor, ids, wts, nullptr,
                                parts)))
     return st;
+  if (path == LayerPath::kFew)
+    return layer_few(s, L, x, x_dtype, residual, T, out, ids, wts, w);
   // shared expert on the GEMV kernels: gate/up from x staged in moe.stage_x
   // (h staged for the down when its format has a packed-f16 kernel), down
   // with the routed rows and the residual folded in
@@ -954,7 +1001,7 @@ int inferno_moe_stack_forward(void* stream, const inferno_moe_layer* layers, siz
     // workgroup of that launch forms the normalised row before its logits
     const inferno_moe_layer* L = &layers[l];
     const bool fused = switch_on("INFERNO_STACK_FUSED_ROUTER") &&
-                       layer_takes_decode(L, T, act_dtype) &&
+                       layer_path(L, T, act_dtype, w.layer_ws) == LayerPath::kDecode &&
                        norm_router_supported(T, H, L->experts, 0);
     int st = fused ? launch_norm_router(s, r, norm_weights[l], eps, L->router, nullptr, T, H,
                                         L->experts, 0, 0, 0, 1.f, act_dtype, w.normed, w.logits,

@@ -28,9 +28,7 @@
 // instead loses a row beside one large value.
 #include "dense_q8.hpp"
 
-#include <cfloat>
-
-#include "gemv_common.hpp"
+#include "scaled_rows.hpp"
 
 namespace inferno {
 namespace {
@@ -59,29 +57,10 @@ __global__ void __launch_bounds__(256)
   const int lane = threadIdx.x & 63, kb = int(blockIdx.y) * 4 + int(threadIdx.x >> 6);
   if (kb * kUnit >= K) return;
   const int at = kb * kUnit + 4 * lane;
-  const uint8_t* src = reinterpret_cast<const uint8_t*>(x + size_t(blockIdx.x) * K + at);
   uint16_t* out = staged + size_t(blockIdx.x) * dense_q8_pitch(K, TERMS);
   float v[4];
-  if constexpr (sizeof(XT) == 2) {
-    const uint2 w = ld_u2(src);
-    v[0] = bits_to_f32(w.x << 16);
-    v[1] = bits_to_f32(w.x & 0xffff0000u);
-    v[2] = bits_to_f32(w.y << 16);
-    v[3] = bits_to_f32(w.y & 0xffff0000u);
-  } else {
-    const uint4 w = ld_u4(src);
-    v[0] = bits_to_f32(w.x);
-    v[1] = bits_to_f32(w.y);
-    v[2] = bits_to_f32(w.z);
-    v[3] = bits_to_f32(w.w);
-  }
-  float m = 0.f;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) m = fabsf(v[j]) <= FLT_MAX ? fmaxf(m, fabsf(v[j])) : m;
-#pragma unroll
-  for (int o = 1; o < 8; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, kWave));
-  const int e = m > 0.f ? 141 - int((f32_to_bits(m) >> 23) & 255u) : 0;
-  // (a subnormal m has exponent field 0: e = 141 puts it below 2^15 all the same)
+  scaled::load4(x + size_t(blockIdx.x) * K + at, v);
+  const int e = scaled::run_exponent<32>(v);
   if ((lane & 7) == 0)
     reinterpret_cast<float*>(out + size_t(TERMS) * K)[kb * 8 + lane / 8] =
         __builtin_amdgcn_ldexpf(1.f, -e);
@@ -92,13 +71,8 @@ __global__ void __launch_bounds__(256)
     hi[j] = (_Float16)u;
     lo[j] = (_Float16)(u - (float)hi[j]);
   }
-  auto put = [&](uint16_t* o, const _Float16* q) {  // k order 0 2 1 3 within four
-    const half2v a = {q[0], q[2]}, b = {q[1], q[3]};
-    *reinterpret_cast<uint2*>(o + at) =
-        make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
-  };
-  put(out, hi);
-  if constexpr (TERMS == 2) put(out + K, lo);
+  scaled::put4(out + at, hi);
+  if constexpr (TERMS == 2) scaled::put4(out + K + at, lo);
 }
 
 // ---------------------------------------------------------------------- GEMM

@@ -68,6 +68,7 @@ struct GemmArgs {
   uint32_t rows;           // dense: number of rows
   int N, K;                // output rows per matrix, reduction length
   uint16_t* h_out;         // two matrices: f16 SwiGLU rows, f16_pitch(N) apart (k order as xin)
+  float* h32;              // two matrices, scaled input rows: fp32 SwiGLU rows [*, N]
   float* y_out;            // one matrix: fp32 rows [*, N]
 };
 
@@ -402,10 +403,11 @@ constexpr int kWaves = 4;
 constexpr int x_halfs(int NB) { return NB == 1 ? 256 : NB == 2 ? 128 : 64; }
 
 // [weights of the four wavefronts][two token buffers][two group-sum buffers]
-template <int Q, int NMAT, int RB, int NB>
+// [two buffers of 16 scales]
+template <int Q, int NMAT, int RB, int NB, bool SCALED>
 constexpr size_t lds_bytes() {
   return size_t(kWaves) * NMAT * RB * 16 * W<Q>::kPitch * 4 + size_t(2) * 16 * NB * x_halfs(NB) * 2 +
-         (W<Q>::kExact ? size_t(2) * NB * 1024 : 0);
+         (W<Q>::kExact ? size_t(2) * NB * 1024 : 0) + (SCALED ? 128 : 0);
 }
 
 // Source of the weight DMA. A wavefront's instruction q copies rows [q RPI,
@@ -476,6 +478,8 @@ struct Lane {
   bool xon[XI];
   uint32_t ssrc;             // group sums: this lane's 16 bytes of unit 0
   bool son;
+  uint32_t csrc;             // scaled rows: this lane's scale of unit 0
+  bool con;
   int xoff;                  // fragment read: byte offset in a token buffer
   int i, g;
 };
@@ -486,10 +490,11 @@ struct Lane {
 // and the LDS read are different buffers, which the restrict qualifiers tell
 // the compiler: it would otherwise wait for the copies before every fragment
 // read.
-template <int Q, int NMAT, int RB, int NB, int SUB>
+template <int Q, int NMAT, int RB, int NB, bool SCALED, int SUB>
 __device__ __forceinline__ void sub_step(const Lane<Q, NMAT, RB, NB>& L, const W<Q>* w, int kb,
                                          bool last, uint8_t* __restrict__ wdst,
                                          uint8_t* __restrict__ xdst, uint8_t* __restrict__ sdst,
+                                         uint8_t* __restrict__ cdst,
                                          const uint8_t* __restrict__ xb, floatx4 (*acc)[NB]) {
   using LN = Lane<Q, NMAT, RB, NB>;
   constexpr int XH = LN::XH, SUBS = kUnit / XH, RT = NMAT * RB;
@@ -500,6 +505,7 @@ __device__ __forceinline__ void sub_step(const Lane<Q, NMAT, RB, NB>& L, const W
     for (int u = 0; u < LN::XI; ++u)
       if (L.xon[u]) dma<16>(L.xin + off, L.xsrc[u], xdst + u * 1024);
     if (W<Q>::kExact && SUB == SUBS - 1 && L.son) dma<16>(L.xin + size_t(kb + 1) * 64, L.ssrc, sdst);
+    if (SCALED && L.con) dma<4>(L.xin + size_t(kb + 1) * 32, L.csrc, cdst);
   }
   if (SUB == (kHalves ? SUBS / 2 : 0) && !last) {
     // behind the tokens: the next buffer's wait leaves the weights in flight
@@ -540,7 +546,7 @@ __device__ __forceinline__ void sub_step(const Lane<Q, NMAT, RB, NB>& L, const W
 
 // The sums of a tile to memory: sum v of lane (i, g) is token 4 g + v of its
 // 16-token block, row i of its 16-row block.
-template <int NMAT, int RB, int NB>
+template <int NMAT, int RB, int NB, bool SCALED>
 __device__ __forceinline__ void store_tile(const GemmArgs& p, const floatx4 (*acc)[NB], uint32_t c0,
                                            uint32_t c1, int n0, int i, int g) {
   uint32_t asg[NB][4];
@@ -567,7 +573,11 @@ __device__ __forceinline__ void store_tile(const GemmArgs& p, const floatx4 (*ac
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         const int r0 = n0 + 16 * rb;
-        if constexpr (NMAT == 2) {
+        if constexpr (NMAT == 2 && SCALED) {
+          if (on)
+            p.h32[size_t(asg[nb][v]) * p.N + r0 + i] =
+                silu(acc[rb][nb][v]) * acc[RB + rb][nb][v] * wts[nb][v];
+        } else if constexpr (NMAT == 2) {
           const _Float16 h = (_Float16)(silu(acc[rb][nb][v]) * acc[RB + rb][nb][v] * wts[nb][v]);
           uint16_t* row = p.h_out + size_t(asg[nb][v]) * f16_pitch(p.N);
           if (on) row[r0 + ip] = __builtin_bit_cast(uint16_t, h);
@@ -586,8 +596,14 @@ __device__ __forceinline__ void store_tile(const GemmArgs& p, const floatx4 (*ac
   }
 }
 
-// OCC: waves per SIMD the registers are budgeted for.
-template <int Q, int NMAT, int RB, int NB, int OCC>
+// OCC: waves per SIMD the registers are budgeted for. SCALED: the input rows
+// are f16_scaled_pitch apart, each 256 of their values in units of their own
+// power of two, which the unit's sums are multiplied by (exactly); h stays
+// fp32. For layers of a few tokens, whose other path (the decode launches)
+// takes activations of any size: plain f16 rows lose h, which grows with the
+// tokens' square, below 1e-3 and above 100 of a token's standard deviation.
+// Four multiplications per 256 values and row block, under 1 % of the launch.
+template <int Q, int NMAT, int RB, int NB, int OCC, bool SCALED = false>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(OCC, 8)))
     wave_gemm_kernel(GemmArgs p) {
   using F = W<Q>;
@@ -602,6 +618,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   constexpr int XI = TM / XROWS / kWaves;  // DMA instructions per wavefront and buffer
   static_assert(XI >= 1 && XI * kWaves * XROWS == TM, "token rows split evenly");
   static_assert(NB <= kWaves, "one group-sum copy per wavefront");
+  static_assert(!SCALED || (NB == 1 && F::kExact), "scales of one token block");
   constexpr int XBUF = TM * XH * 2;
   constexpr int WREG = RT * 16 * F::kPitch * 4;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_g[];
@@ -616,6 +633,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   uint8_t* const wl = smem_g + wave * WREG;
   uint8_t* const xl = smem_g + kWaves * WREG;
   uint8_t* const sl = xl + 2 * XBUF;
+  uint8_t* const cl = sl + 2 * NB * 1024;  // SCALED only
+  const size_t pitch = SCALED ? f16_scaled_pitch(K) : f16_pitch(K);
 
   Lane<Q, NMAT, RB, NB> L;
   L.i = i;
@@ -636,7 +655,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   auto row_off = [&](int r) {
     const uint32_t cc = min(c0 + uint32_t(r), c1 - 1);
     const uint32_t a = p.sorted ? p.sorted[cc] : cc;
-    return (a / p.in_div) * uint32_t(f16_pitch(K)) * 2u;
+    return (a / p.in_div) * uint32_t(pitch) * 2u;
   };
 #pragma unroll
   for (int u = 0; u < XI; ++u) {
@@ -647,6 +666,9 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   // group sums: wavefront nb copies those of token block nb, 64 bytes a row
   L.son = wave < NB && c0 + uint32_t(16 * wave + (lane >> 2)) < c1;
   L.ssrc = row_off(16 * wave + (lane >> 2)) + uint32_t(K) * 2u + 16 * (lane & 3);
+  // scales: wavefront 1 copies one of each row (a unit's eight are equal)
+  L.con = SCALED && wave == 1 && lane < 16 && c0 + uint32_t(lane) < c1;
+  L.csrc = SCALED ? row_off(lane & 15) + uint32_t(f16_scale_at(K)) * 2u : 0u;
   L.xin = reinterpret_cast<const uint8_t*>(p.xin);
   L.xoff = i * XH * 2 + 16 * (g ^ swz(i));
 
@@ -662,6 +684,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   for (int u = 0; u < XI; ++u)
     if (L.xon[u]) dma<16>(L.xin, L.xsrc[u], xw + u * 1024);
   if (F::kExact && L.son) dma<16>(L.xin, L.ssrc, sl + wave * 1024);
+  if (SCALED && L.con) dma<4>(L.xin, L.csrc, cl);
   constexpr int NW = NMAT * ((RM + WSrc<Q>::RPI - 1) / WSrc<Q>::RPI);  // weight DMAs per unit
   // up to 32 tokens: the whole super-block of every row in registers, the
   // region refilled at once; above, one half at a time beside the sums
@@ -670,6 +693,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
   W<Q> w[kHalves ? RT : 2 * RT];
   float ds[RT];
   floatx4 part[F::kExact ? RT : 1][NB];  // the unit's sums, in units of its d
+  floatx4 offs[SCALED ? RT : 1], cs;     // SCALED: its offset terms, the tokens' scales
   const uint32_t* const wrd = reinterpret_cast<const uint32_t*>(wl) + i * F::kPitch;
   for (int kb = 0; kb < nkb; ++kb) {
     const bool last = kb + 1 == nkb;
@@ -690,6 +714,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
       asm volatile("" ::: "memory");
       if constexpr (F::kExact && S == 0) {
         // the unit's offset terms: their integers times the group sums
+        if constexpr (SCALED) cs = *reinterpret_cast<const floatx4*>(cl + (kb & 1) * 64 + g * 16);
         const uint8_t* sb = sl + (kb & 1) * (NB * 1024) + i * 64 + g * 16;
         half8 xs[NB];
 #pragma unroll
@@ -705,7 +730,8 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             const floatx4 m = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                 xs[nb], o, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
             if constexpr (F::kMin) {
-              acc[r][nb] += m * ms;
+              if constexpr (SCALED) offs[r] = m * ms;
+              else acc[r][nb] += m * ms;
               part[r][nb] = floatx4{0.f, 0.f, 0.f, 0.f};
             } else {
               part[r][nb] = m;
@@ -732,8 +758,9 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
       }
       // the words are in registers: the region is free for the next unit
       if constexpr (S == WS) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      sub_step<Q, NMAT, RB, NB, S>(L, w, kb, last, wl, xw + (bufof(S) ^ 1) * XBUF,
+      sub_step<Q, NMAT, RB, NB, SCALED, S>(L, w, kb, last, wl, xw + (bufof(S) ^ 1) * XBUF,
                                    sl + ((kb & 1) ^ 1) * (NB * 1024) + wave * 1024,
+                                   cl + ((kb & 1) ^ 1) * 64,
                                    xl + bufof(S) * XBUF, F::kExact ? part : acc);
     };
     sub(std::integral_constant<int, 0>{});
@@ -746,10 +773,15 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[r][nb] += part[r][nb] * ds[r];
+        for (int nb = 0; nb < NB; ++nb) {
+          if constexpr (SCALED)
+            acc[r][nb] += (F::kMin ? part[r][nb] * ds[r] + offs[r] : part[r][nb] * ds[r]) * cs;
+          else
+            acc[r][nb] += part[r][nb] * ds[r];
+        }
     }
   }
-  store_tile<NMAT, RB, NB>(p, acc, c0, c1, n0, i, g);
+  store_tile<NMAT, RB, NB, SCALED>(p, acc, c0, c1, n0, i, g);
 }
 
 }  // namespace grouped

@@ -34,6 +34,7 @@
 #include "grouped_gemm.hpp"
 #include "grouped_gemm128.hpp"
 #include "routing_dev.hpp"
+#include "scaled_rows.hpp"
 
 namespace inferno {
 namespace {
@@ -903,6 +904,37 @@ __global__ void __launch_bounds__(256)
   reinterpret_cast<uint16_t*>(row)[f16_sum_at(K, c8 / 2, term)] = f16_sum_term(t, term);
 }
 
+// Scaled rows of two matrices in one launch: blockIdx.x is a row of the first,
+// then of the second; a wavefront per 256 values.
+template <typename XT>
+__global__ void __launch_bounds__(256) scaled_rows_kernel(RowsToScale r0, RowsToScale r1) {
+  const bool second = blockIdx.x >= r0.rows;
+  const RowsToScale& m = second ? r1 : r0;
+  const size_t row = second ? blockIdx.x - r0.rows : blockIdx.x, K = m.K;
+  const uint32_t lane = threadIdx.x & 63, kb = blockIdx.y * 4 + (threadIdx.x >> 6);
+  if (size_t(kb) * kUnit >= K) return;  // a whole wavefront
+  const size_t at = size_t(kb) * kUnit + 4 * lane;
+  uint16_t* out = m.out + row * f16_scaled_pitch(K);
+  float v[4];
+  scaled::load4(static_cast<const XT*>(m.x) + row * K + at, v);
+  const int e = scaled::run_exponent<kUnit>(v);
+  _Float16 q[4];
+  float t = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    q[j] = (_Float16)__builtin_amdgcn_ldexpf(v[j], e);
+    t += (float)q[j];
+  }
+  scaled::put4(out + at, q);
+  t += __shfl_xor(t, 1, kWave);  // the group of 16: four lanes
+  t += __shfl_xor(t, 2, kWave);
+  if ((lane & 3) < 2)
+    out[f16_sum_at(K, 16 * size_t(kb) + lane / 4, int(lane & 3))] = f16_sum_term(t, int(lane & 3));
+  if (lane < 8)
+    reinterpret_cast<float*>(out + f16_scale_at(K))[8 * size_t(kb) + lane] =
+        __builtin_amdgcn_ldexpf(1.f, -e);
+}
+
 // out = (residual + ys) + y ranks 0..k-1 of the token, in that order; one
 // float4 per thread. The k rank rows are loaded at once (KMAX slots, the
 // indices clamped to k - 1 and the extra slots not added), so a wavefront
@@ -1113,17 +1145,20 @@ PlanView plan_view(uint32_t* plan, size_t A, size_t E, bool narrow) {
 // True when the LDS DMA can stage the GEMM's operands: matrices and input
 // rows aligned to the piece it moves per lane, whole workgroups of rows, and
 // input rows within the 32-bit offset of a lane.
+bool dma_takes(int quant, const void* w0, const void* w1, const void* rows, size_t N) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(w0) | reinterpret_cast<uintptr_t>(w1);
+  return p % (quant == INFERNO_Q4_K ? 16 : 4) == 0 && N % 256 == 0 &&
+         reinterpret_cast<uintptr_t>(rows) % 16 == 0;
+}
 bool wave_gemm_takes(int quant, const GemmArgs& a) {
-  const uintptr_t p = reinterpret_cast<uintptr_t>(a.w0) | reinterpret_cast<uintptr_t>(a.w1);
-  return p % (quant == INFERNO_Q4_K ? 16 : 4) == 0 && a.N % 256 == 0 &&
-         reinterpret_cast<uintptr_t>(a.xin) % 16 == 0 &&
+  return dma_takes(quant, a.w0, a.w1, a.xin, size_t(a.N)) &&
          a.in_rows * f16_pitch(a.K) * 2 <= size_t(0xffffffffu);
 }
 
-template <int Q, int NMAT, int RB, int NB, int OCC>
+template <int Q, int NMAT, int RB, int NB, int OCC, bool SCALED = false>
 int launch_wave_gemm(hipStream_t s, const GemmArgs& a, unsigned grid_y) {
-  constexpr size_t lds = grouped::lds_bytes<Q, NMAT, RB, NB>();
-  auto kern = grouped::wave_gemm_kernel<Q, NMAT, RB, NB, OCC>;
+  constexpr size_t lds = grouped::lds_bytes<Q, NMAT, RB, NB, SCALED>();
+  auto kern = grouped::wave_gemm_kernel<Q, NMAT, RB, NB, OCC, SCALED>;
   static_assert(lds <= 64 * 1024, "within the default dynamic LDS limit");
   const dim3 grid(unsigned(a.N / (16 * RB * grouped::kWaves)), grid_y);
   kern<<<grid, 256, lds, s>>>(a);
@@ -1143,6 +1178,22 @@ int launch_wave_q(hipStream_t s, int quant, const GemmArgs& a, unsigned grid_y) 
       break;
   }
   set_error("quant kind has no grouped GEMM");
+  return INFERNO_ERR_INVALID;
+}
+
+// The GEMMs of a few tokens (scaled rows): 16-row tiles.
+template <int NMAT>
+int launch_few(hipStream_t s, int quant, GemmArgs a, const PlanView& v) {
+  constexpr int RB = NMAT == 2 ? 1 : 2;
+  a.tiles = v.l16;
+  a.n_tiles = v.counts + 3;
+  const unsigned gy = unsigned(v.n16);
+  switch (quant) {
+    case INFERNO_Q2_K: return launch_wave_gemm<INFERNO_Q2_K, NMAT, RB, 1, 4, true>(s, a, gy);
+    case INFERNO_Q3_K: return launch_wave_gemm<INFERNO_Q3_K, NMAT, RB, 1, 4, true>(s, a, gy);
+    case INFERNO_Q4_K: return launch_wave_gemm<INFERNO_Q4_K, NMAT, RB, 1, 4, true>(s, a, gy);
+  }
+  set_error("quant kind has no grouped GEMM of scaled rows");
   return INFERNO_ERR_INVALID;
 }
 
@@ -1276,6 +1327,26 @@ size_t prefill_plan_words(size_t A, size_t E) {
   return 4 * (bound128(A, E) + 2 * bound_small(A, E) + bound16(A, E, true)) + 4;
 }
 
+int launch_scaled_rows(hipStream_t s, int x_dtype, const RowsToScale& r0, const RowsToScale& r1) {
+  const size_t rows = r0.rows + r1.rows, K = std::max(r0.K, r1.rows ? r1.K : 0);
+  if (rows == 0) return INFERNO_OK;
+  if (r0.K % kUnit || (r1.rows && r1.K % kUnit) || rows > 0x7fffffffu || K / kUnit / 4 >= 65535) {
+    set_error("scaled rows: widths of a multiple of 256");
+    return INFERNO_ERR_INVALID;
+  }
+  const dim3 grid{unsigned(rows), unsigned((K / kUnit + 3) / 4)};
+  if (x_dtype == INFERNO_BF16) scaled_rows_kernel<uint16_t><<<grid, 256, 0, s>>>(r0, r1);
+  else scaled_rows_kernel<float><<<grid, 256, 0, s>>>(r0, r1);
+  INF_LAUNCHED();
+  return INFERNO_OK;
+}
+
+bool prefill_few_takes(int quant, int down_quant, const void* gate, const void* up,
+                       const void* down, const void* rows, size_t H, size_t I, size_t E) {
+  return down_quant != INFERNO_Q6_K && prefill_routed_supported(quant, down_quant, H, I, E) &&
+         dma_takes(quant, gate, up, rows, I) && dma_takes(down_quant, down, nullptr, rows, H);
+}
+
 int launch_to_f16(hipStream_t s, const void* x, int x_dtype, size_t rows, size_t K,
                   uint16_t* out) {
   const size_t n8 = rows * K / 8;
@@ -1310,6 +1381,7 @@ GemmArgs gate_up_args(const PrefillRouted& p) {
   g.N = int(p.I);
   g.K = int(p.H);
   g.h_out = p.h16;
+  g.h32 = p.h32;
   return g;
 }
 GemmArgs down_args(const PrefillRouted& p) {
@@ -1350,7 +1422,7 @@ constexpr size_t kNarrowRows = 10;
 constexpr size_t kNarrowGroups = 2560;
 bool narrow_layer(const PrefillRouted& p) {
   const size_t A = p.T * p.k;
-  return A <= kNarrowRows * p.E ||
+  return p.h32 != nullptr || A <= kNarrowRows * p.E ||
          (wave_layer(p) && (p.E + A / 16) * (p.I / 64) <= kNarrowGroups);
 }
 }  // namespace
@@ -1369,6 +1441,7 @@ int launch_prefill_gate_up(hipStream_t s, const PrefillRouted& p) {
     return INFERNO_ERR_INVALID;
   }
   const bool narrow = narrow_layer(p);
+  if (p.h32) return launch_few<2>(s, p.quant, gate_up_args(p), plan_view(p.plan, A, p.E, narrow));
   return launch_tiled<2>(s, p.quant, gate_up_args(p), plan_view(p.plan, A, p.E, narrow),
                          p.max_rows ? p.max_rows : A, narrow, wave_layer(p));
 }
@@ -1377,6 +1450,7 @@ int launch_prefill_down(hipStream_t s, const PrefillRouted& p) {
   const size_t A = p.T * p.k;
   if (A == 0) return INFERNO_OK;
   const bool narrow = narrow_layer(p);
+  if (p.h32) return launch_few<1>(s, p.down_quant, down_args(p), plan_view(p.plan, A, p.E, narrow));
   return launch_tiled<1>(s, p.down_quant, down_args(p), plan_view(p.plan, A, p.E, narrow),
                          p.max_rows ? p.max_rows : A, narrow, wave_layer(p));
 }

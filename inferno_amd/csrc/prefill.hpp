@@ -18,21 +18,21 @@ bool prefill_routed_supported(int quant, int down_quant, size_t H, size_t I, siz
 // against 1.015, T = 8 1.151 against 1.050, c2 T = 10 0.408 against 0.378).
 constexpr size_t kPrefillMinAssignments = 48;
 constexpr size_t kPrefillMinAssignmentsShared = 66;
-// Several tokens below those counts, in a layer that the fused decode launches
-// also take: the grouped GEMMs when the assignments' expert bytes outweigh
-// their more launches (seven against four, two more with a shared expert).
-// Measured over H 1024 .. 6144, I 512 .. 2048, Q2_K / Q3_K / Q4_K, decode /
-// grouped in us: without a shared expert 2048 x 768 Q4_K 16 assignments 39 /
-// 34, 24 47 / 41; 2816 x 1280 Q2_K 16 48 / 50, 18 51 / 50, 24 61 / 52; 1024 x
-// 512 Q2_K 18 (9 MB) 29 / 29, 32 (17 MB) 33 / 29; with one 4096 x 1536 Q2_K 16
-// (99 MB) 63 / 66, 24 77 / 73, 32 96 / 83; 6144 x 2048 Q2_K 16 (198 MB) 101 /
-// 99, 32 177 / 143; 2048 x 768 Q2_K 32 (50 MB) 44 / 47. A narrow expert under
-// a wide row (6144 x 512: few workgroups, each with a long K) needs more:
-// Q2_K 18 50 / 57, 24 61 / 59, with a shared expert Q4_K 24 64 / 68, 32 78 / 70.
-inline bool grouped_beats_decode(size_t A, size_t H, size_t I, size_t expert_bytes, bool shared) {
-  const bool narrow = H > 4 * I;
-  return shared ? A >= (narrow ? 32 : 16) && A * expert_bytes >= size_t(100) << 20
-                : A >= (narrow ? 24 : 18) && A * expert_bytes >= size_t(14) << 20;
+// Several bf16 tokens below those counts, in a layer that the fused decode
+// launches also take: the grouped GEMMs over scaled rows when the assignments'
+// expert bytes outweigh their launches (nine against four, three of them short
+// ones that the decode launches have no counterpart of; two more with a shared
+// expert). Measured over 28 layers (H 1024 .. 6144, I 512 .. 2048, Q2_K / Q3_K /
+// Q4_K, with and without a shared expert) of 2 to 8 tokens, decode / grouped in
+// us: from 24 assignments and 130 MiB on at worst 1.5 % slower, 19 % faster on
+// average (68 points; Q2_K H 6144 I 2048 24 assignments, 284 MiB 115 / 116,
+// with a shared expert 32 of them 378 MiB 177 / 153; Q4_K H 2816 I 1280 24,
+// 139 MiB 62 / 56; Q3_K H 4096 I 1536 40, 309 MiB 146 / 126), below it mostly
+// slower (Q2_K H 4096 I 1536 20, 118 MiB 65 / 68; Q3_K H 2048 I 768 32, 62 MiB
+// 50 / 53; Q4_K H 6144 I 512 24, 122 MiB 61 / 63; Q2_K H 6144 I 2048 16, 189
+// MiB 85 / 92).
+inline bool grouped_beats_decode(size_t A, size_t expert_bytes) {
+  return A >= 24 && A * expert_bytes >= size_t(130) << 20;
 }
 
 // 32-bit words of the routed planner's scratch (tile lists and counts).
@@ -58,6 +58,21 @@ __device__ __forceinline__ uint16_t f16_sum_term(float t, int term) {
   return __builtin_bit_cast(uint16_t, term == 0 ? hi : (_Float16)((m - (float)hi) * 2048.0f));
 }
 
+// Scaled rows (the grouped GEMMs of a few tokens): the same, with the values in
+// units of a power of two per 256 of them, and behind the padding a fp32 per 32
+// values, eight equal ones per unit, that brings sums back.
+HD constexpr size_t f16_scale_at(size_t K) { return f16_pitch(K); }
+HD constexpr size_t f16_scaled_pitch(size_t K) { return f16_pitch(K) + K / 16; }
+
+// rows0 [n0, K0] and, unless n1 is 0, rows1 [n1, K1] (bf16 or fp32) as scaled
+// rows, in one launch.
+struct RowsToScale {
+  const void* x;
+  uint16_t* out;  // f16_scaled_pitch(K) apart, 8-byte aligned
+  size_t rows, K;
+};
+int launch_scaled_rows(hipStream_t s, int x_dtype, const RowsToScale& r0, const RowsToScale& r1);
+
 // x [rows, K] (bf16 or fp32) -> f16 rows of f16_pitch(K), round to nearest even.
 int launch_to_f16(hipStream_t s, const void* x, int x_dtype, size_t rows, size_t K, uint16_t* out);
 
@@ -76,7 +91,14 @@ struct PrefillRouted {
   // most rows one expert can take: T when every token's ids are distinct
   // (the layer's own top-k), 0 when unknown (caller ids: up to A)
   size_t max_rows;
+  // a few tokens (prefill_few_takes): x16 and h16 are scaled rows, the gate/up
+  // writes h32 [A, I] for launch_scaled_rows to turn into h16; else null
+  float* h32;
 };
+// True when the scaled-row GEMMs take a layer: formats, widths and the
+// alignment of the weights and of the rows.
+bool prefill_few_takes(int quant, int down_quant, const void* gate, const void* up,
+                       const void* down, const void* rows, size_t H, size_t I, size_t E);
 
 // The tile lists of the layer inside p.plan, for the dispatch launch to fill
 // (launch_dispatch with a plan) before launch_prefill_gate_up reads them.

@@ -1,5 +1,7 @@
 """Layers of a few tokens, on both sides of the rule that hands them from the
-fused decode launches to the grouped GEMMs."""
+fused decode launches to the grouped GEMMs: tokens of any size (h grows with
+their square, so that plain f16 rows would lose it at either end), one
+activation far above the others, fp32 tokens, more than one tile of rows."""
 import pytest
 import torch
 
@@ -12,7 +14,7 @@ def _weights(quant, seed, rows, cols):
     return ops.synth_quantized(quant, seed, 0.02, rows, cols, torch.device("cuda:0"))
 
 
-def _layer(quant, shared, T, router_std=0.02):
+def _layer(quant, shared, T, router_std=0.02, E=E, k=TOP_K):
     g = torch.Generator(device="cuda").manual_seed(2)
     kw = {}
     if shared:
@@ -21,7 +23,7 @@ def _layer(quant, shared, T, router_std=0.02):
     mats = dict(gate=_weights(quant, 0, E * I, H), up=_weights(quant, 1, E * I, H),
                 down=_weights(quant, 2, E * H, I))
     layer = ops.MoELayer(
-        hidden=H, experts=E, intermediate=I, top_k=TOP_K, quant=quant, down_quant=quant,
+        hidden=H, experts=E, intermediate=I, top_k=k, quant=quant, down_quant=quant,
         score_fn=SCORE_SOFTMAX, norm_topk_prob=True, routed_scaling_factor=1.0,
         router=torch.randn(E, H, generator=g, device="cuda") * router_std, router_bias=None,
         shared_intermediate=IS if shared else 0, max_tokens=T, **mats, **kw)
@@ -30,7 +32,7 @@ def _layer(quant, shared, T, router_std=0.02):
 
 def _exact(quant, mats, kw, x, ids, w):
     """The layer in 64 bits for the ids and weights that the layer chose."""
-    deq = {n: ops.dequantize(quant, m).view(E, -1, I if n == "down" else H).double()
+    deq = {n: ops.dequantize(quant, m).view(-1, *((H, I) if n == "down" else (I, H))).double()
            for n, m in mats.items()}
     x = x.double()
 
@@ -48,27 +50,69 @@ def _exact(quant, mats, kw, x, ids, w):
     return out
 
 
-def _both_sides(quant, shared, x, monkeypatch, **kw):
-    """Relative error of each token's row against fp64, by the rule and on the
-    decode launches (a threshold that no batch reaches)."""
+def _sides(monkeypatch, layer, x):
+    """The layer by the rule, on the decode launches, on the grouped GEMMs."""
+    out = [layer.forward(x)]
+    for side in ("0", "1"):
+        monkeypatch.setenv("INFERNO_DECODE_GROUPED", side)
+        out.append(layer.forward(x))
+    monkeypatch.delenv("INFERNO_DECODE_GROUPED")
+    return out
+
+
+def _row_errors(monkeypatch, quant, shared, x, **kw):
+    """Largest error of a token's row against fp64: decode, grouped."""
     T = x.shape[0]
     layer, mats, sh = _layer(quant, shared, T, **kw)
-    ids = torch.empty(T * TOP_K, dtype=torch.int32, device="cuda")
-    w = torch.empty(T * TOP_K, device="cuda")
-    by_rule = layer.forward(x, None, ids=ids, weights=w)
-    ref = _exact(quant, mats, sh, x, ids.view(T, TOP_K), w.view(T, TOP_K))
-    monkeypatch.setenv("INFERNO_PREFILL_MIN_ASSIGNMENTS", "100000")
-    decode = layer.forward(x)
-
-    def err(y):
-        return ((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).max().item()
-
-    return err(by_rule), err(decode), by_rule, decode
+    ids = torch.empty(T * layer.top_k, dtype=torch.int32, device="cuda")
+    w = torch.empty(T * layer.top_k, device="cuda")
+    layer.forward(x, None, ids=ids, weights=w)
+    ref = _exact(quant, mats, sh, x, ids.view(T, -1), w.view(T, -1))
+    _, decode, grouped = _sides(monkeypatch, layer, x)
+    assert not torch.equal(decode, grouped)  # two paths ran
+    return [((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).max().item()
+            for y in (decode, grouped)]
 
 
-# The decode launches round weights times scales and h to f16, in units that
-# each 16 values choose; per row (the layers' own 2e-3 is per batch).
-BOUND = 2e-3
+# Grouped: f16 holds bf16 tokens and the integers of the weights, so that what
+# is rounded is h, by at most 2^-11 of each value. Decode: the products of
+# weights and scales too (the layers' own bound).
+GROUPED, DECODE = 2.0 ** -11, 2e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [2, 4, 6])
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("quant", [Q2_K, Q3_K, Q4_K])
+@pytest.mark.parametrize("scale", [1e-3, 0.02, 1.0, 200.0])
+def test_token_scale(quant, shared, T, scale, monkeypatch):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = (torch.randn(T, H, generator=g, device="cuda") * scale).bfloat16()
+    decode, grouped = _row_errors(monkeypatch, quant, shared, x, router_std=1e-4)
+    assert grouped < GROUPED and decode < DECODE, (grouped, decode)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [2, 6])
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("quant", [Q2_K, Q3_K, Q4_K])
+def test_one_large_activation(quant, shared, T, monkeypatch):
+    # 1e5 in one token (past f16's range); a router of 1e-6 hardly sees it
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(T, H, generator=g, device="cuda")
+    x[T - 1, 5] = 1e5
+    decode, grouped = _row_errors(monkeypatch, quant, shared, x.bfloat16(), router_std=1e-6)
+    assert grouped < GROUPED and decode < DECODE, (grouped, decode)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant", [Q2_K, Q3_K, Q4_K])
+def test_more_than_one_tile(quant, monkeypatch):
+    # 40 tokens over two experts: tiles of 16 rows and a remainder of each
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(40, H, generator=g, device="cuda").bfloat16()
+    decode, grouped = _row_errors(monkeypatch, quant, True, x, E=2, k=1)
+    assert grouped < GROUPED and decode < DECODE, (grouped, decode)
 
 
 @pytest.mark.gpu
@@ -80,5 +124,22 @@ def test_fp32_tokens_keep_their_bits(quant, shared, T, monkeypatch):
     # term of the grouped GEMMs would hold 11, so the rule leaves them there
     g = torch.Generator(device="cuda").manual_seed(3)
     x = torch.randn(T, H, generator=g, device="cuda")
-    _, decode, y, z = _both_sides(quant, shared, x, monkeypatch)
-    assert decode < BOUND and torch.equal(y, z)
+    layer, _, _ = _layer(quant, shared, T)
+    by_rule, decode, forced = _sides(monkeypatch, layer, x)
+    assert torch.equal(by_rule, decode) and torch.equal(forced, decode)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("quant,T,hands_over", [
+    (Q3_K, 3, False),  # 18 assignments
+    (Q2_K, 6, False),  # 36 assignments of 110 MiB
+    (Q3_K, 6, True),   # 145 MiB
+    (Q4_K, 5, True)])  # 158 MiB
+def test_rule(quant, T, hands_over, shared, monkeypatch):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    layer, _, _ = _layer(quant, shared, T)
+    by_rule, decode, grouped = _sides(monkeypatch, layer, x)
+    assert not torch.equal(decode, grouped)
+    assert torch.equal(by_rule, grouped if hands_over else decode)
