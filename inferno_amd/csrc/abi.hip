@@ -2,6 +2,7 @@
 // Err paths, e.g. crates/backend/src/metal/gguf_moe.rs:84-121 and
 // crates/backend/src/metal/moe.rs:582-623), workspace carving and kernel
 // sequencing. No function allocates device memory or synchronises.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -65,8 +66,8 @@ struct MoeScratch {
   float* h;
   float* y;
   uint32_t* stage_x;  // staged activations of x (sized for fp32 input); f16 x on the MFMA path
-  uint32_t* stage_h;  // staged activations of h
-  uint32_t* plan;     // MFMA path: expert tile lists
+  uint32_t* stage_h;  // staged activations of h; scaled rows of h (a few tokens)
+  uint32_t* plan;     // grouped GEMMs: expert tile lists, at the end of stage_h
 };
 
 // Staged activation rows, sized for the fp32 (split) layout, the larger one.
@@ -83,8 +84,11 @@ MoeScratch carve_moe(Carver& c, size_t T, size_t k, size_t E, size_t H, size_t I
   m.y = c.take<float>(T * k * H);
   m.stage_x = c.take<uint32_t>(stage_words(T, H));
   // (one row more: the shared expert's h when it runs as assignment k)
-  m.stage_h = c.take<uint32_t>(stage_words(T * k + 1, I));
-  m.plan = c.take<uint32_t>(prefill_plan_words(T * k, E));
+  const size_t words = stage_words(T * k + 1, I);
+  m.stage_h = c.take<uint32_t>(words);
+  // the grouped GEMMs leave the region's end free: scaled rows take 2.4 I + 128
+  // of its 4.5 I bytes per row, the lists at most 50
+  m.plan = m.stage_h + (words - std::min(words, prefill_plan_words(T * k, E))) / 4 * 4;
   return m;
 }
 
@@ -522,6 +526,7 @@ int inferno_rms_norm_router_topk(void* stream, const float* x, const float* norm
 namespace {
 struct LayerScratch {
   float* logits;
+  size_t logits_parts;  // the chunks of them that fit
   uint32_t* ids;
   float* weights;
   float* hs;
@@ -542,14 +547,16 @@ struct LayerScratch {
 // the no-alloc entry point passes false: the library allocates on its own.
 LayerScratch carve_layer(Carver& c, const inferno_moe_layer* L, size_t T, bool lib = true) {
   LayerScratch s;
-  // router logits, or their K-chunk partials for a small bf16 batch
-  s.logits = c.take<float>(T * L->experts *
-                           size_t(router_logit_parts_max(T, L->hidden, L->experts)));
   s.ids = c.take<uint32_t>(T * L->top_k);
   s.weights = c.take<float>(T * L->top_k);
   s.hs = c.take<float>(T * (L->shared_intermediate ? L->shared_intermediate : 1));
   s.stage_hs = c.take<uint32_t>(L->shared_intermediate ? stage_words(T, L->shared_intermediate) : 1);
   s.moe = carve_moe(c, T, L->top_k, L->experts, L->hidden, L->intermediate);
+  // router logits, or their K-chunk partials for a small batch: read by the
+  // top-k, before the down rows are written over them. (So the need is linear
+  // in T: the number of chunks is not, it falls as T grows.)
+  s.logits_parts = std::max<size_t>(1, L->top_k * L->hidden / std::max<size_t>(1, L->experts));
+  s.logits = L->top_k * L->hidden >= L->experts ? s.moe.y : c.take<float>(T * L->experts);
   s.partials = c.take<float>(size_t(L->hidden / decode_chunk(L->hidden)) * T * L->experts);
   s.ys = c.take<float>(T * L->hidden);
   s.slots = c.take<uint4>(L->experts);
@@ -798,7 +805,7 @@ int layer_forward(void* stream, const inferno_moe_layer* L, const void* x, int x
   // router's three bf16 terms
   const bool router_blas = w.rblas != nullptr && w.blas_lib != nullptr &&
                            router_blas_takes(T, H, E, x_dtype);
-  const int parts = router_blas ? 1 : router_logit_parts(T, H, E, x_dtype);
+  const int parts = router_blas ? 1 : router_logit_parts(T, H, E, x_dtype, w.logits_parts);
   const bool mfma_path = path == LayerPath::kGrouped;
   // the shared expert on the dense MFMA GEMMs when its formats have them
   // (Q8_0; the Laguna XS Q4_K gate/up with Q4_K or Q6_K down), else on the

@@ -18,11 +18,9 @@ int launch_router_topk(hipStream_t s, const float* logits, const float* bias, si
                        size_t k, int score_fn, int norm, float scale, uint32_t* ids,
                        float* weights, uint32_t* token_idx, int parts = 1);
 // Router logits of bf16 tokens split over K chunks for small batches (more
-// workgroups): router_logit_parts() chunks of partials [parts][T][E], summed
-// by launch_router_topk(..., parts); router_logit_parts_max() bounds it for
-// any token type and switch setting (workspace sizing).
-int router_logit_parts(size_t T, size_t H, size_t E, int x_dtype);
-int router_logit_parts_max(size_t T, size_t H, size_t E);
+// workgroups): router_logit_parts() chunks of partials [parts][T][E], at most
+// `most`, summed by launch_router_topk(..., parts).
+int router_logit_parts(size_t T, size_t H, size_t E, int x_dtype, size_t most);
 // True when the K-chunk logits launch of fp32 tokens (parts > 1) can also
 // write x in f16 (the grouped GEMMs' copy, as launch_to_f16 writes it).
 bool router_writes_x16(size_t T, size_t H, size_t E, int x_dtype, int parts);

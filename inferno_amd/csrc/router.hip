@@ -8,6 +8,7 @@
 // holds up to four candidates and each round is a DPP wavefront max of the
 // order-preserving key, then of ~expert id among the lanes holding that key
 // (routing_dev.hpp).
+#include <algorithm>
 #include <cstdlib>
 
 #include "prefill.hpp"
@@ -417,24 +418,20 @@ static bool bf16x3_enabled() {
 // kMaxRouterParts) that keeps at most kRouterSplitGroups workgroups of the
 // one-group kernel and a whole number of 32-deep block pairs per chunk. Any
 // divisor of the pairs: H 2816 takes 11 chunks (a power of two gave it 4 and
-// the launch 15.4 us instead of 7.3).
+// the launch 15.4 us instead of 7.3). At most `most`: what the caller's region
+// for the partials holds.
 constexpr size_t kRouterSplitGroups = 256;
-int router_logit_parts_max(size_t T, size_t H, size_t E) {
-  if (H % 256) return 1;
+int router_logit_parts(size_t T, size_t H, size_t E, int x_dtype, size_t most) {
+  if (H % 256 || (x_dtype == INFERNO_BF16 && !bf16x3_enabled())) return 1;
   const size_t base = ((E + 63) / 64) * ((T + 15) / 16);
   if (base * 2 > kRouterSplitGroups) return 1;
-  int z = kMaxRouterParts;
+  int z = int(std::max<size_t>(1, std::min<size_t>(kMaxRouterParts, most)));
   while (z > 1 && (base * size_t(z) > kRouterSplitGroups || (H / 64) % size_t(z) != 0)) --z;
   return z;
 }
 bool router_writes_x16(size_t T, size_t H, size_t E, int x_dtype, int parts) {
   (void)T; (void)E;
   return parts > 1 && H % 32 == 0;
-}
-
-int router_logit_parts(size_t T, size_t H, size_t E, int x_dtype) {
-  if (x_dtype == INFERNO_BF16 && !bf16x3_enabled()) return 1;
-  return router_logit_parts_max(T, H, E);
 }
 
 int launch_router_logit_parts(hipStream_t s, const void* x, int x_dtype, const float* w, size_t T,
