@@ -1229,7 +1229,10 @@ int launch_tile128_q(hipStream_t s, int quant, const GemmArgs& a, unsigned grid_
 // 65 rows, no 64-row tile below 33) is not launched; its grid of workgroups
 // that find no tile would still take a few microseconds. wave: the DMA
 // kernels take the operands (measured in grouped_gemm.hpp for tiles of up to
-// 64 rows, in grouped_gemm128.hpp for the others).
+// 64 rows, in grouped_gemm128.hpp for the others). The general kernels' tiles
+// have at least 32 rows: a list of 16-row remainders would half fill them and
+// cost a launch per GEMM (64 experts of 768 x 2048, 2048 assignments: Q2_K 115
+// -> 145 us, Q4_K 161 -> 195).
 template <int NMAT>
 int launch_tiled(hipStream_t s, int quant, GemmArgs a, const PlanView& v, size_t max_rows,
                  bool narrow, bool wave) {
@@ -1247,8 +1250,8 @@ int launch_tiled(hipStream_t s, int quant, GemmArgs a, const PlanView& v, size_t
       return st;
     a.tiles = v.l32;
     a.n_tiles = v.counts + 2;
-    if (max_rows > 16 && (st = wave ? launch_wave_q<NMAT, 2, 4>(s, quant, a, unsigned(v.n32))
-                                    : launch_gemm_q<NMAT, 32>(s, quant, a, unsigned(v.n32))))
+    if (!wave) return launch_gemm_q<NMAT, 32>(s, quant, a, unsigned(v.n32));
+    if (max_rows > 16 && (st = launch_wave_q<NMAT, 2, 4>(s, quant, a, unsigned(v.n32))))
       return st;
   }
   a.tiles = v.l16;
@@ -1411,6 +1414,9 @@ bool wave_layer(const PrefillRouted& p) {
 // experts (2 rows each) 61 -> 52 us, 64 tokens (8 rows) 125 -> 118 us; 32
 // tokens x 10 over 128 experts even; H 6144, I 2048, 256 experts of 8 rows,
 // Q2_K 907 -> 760 us, Q3_K 1060 -> 990, of 11 rows 950 -> 905, 1110 -> 1200.
+// The general kernels, which half fill their 32-row tiles: 64 experts of 768 x
+// 2048, 256 assignments, Q2_K 74 -> 66, Q3_K 81 -> 75, Q4_K 76 -> 70 us, 512
+// 73 -> 70, 80 -> 74, 77 -> 76; 256 experts of 2048 x 6144, 512 even.
 // On the DMA kernels also while those tiles make at most 2560 gate/up
 // workgroups (four per CU at a time): whole layers, all tile sizes -> 16-row
 // tiles only: H 2048, I 768, 64 experts, Q4_K, 704 assignments (1296
@@ -1430,7 +1436,7 @@ bool narrow_layer(const PrefillRouted& p) {
 PlanOut prefill_plan_out(const PrefillRouted& p) {
   const bool narrow = narrow_layer(p);
   const PlanView v = plan_view(p.plan, p.T * p.k, p.E, narrow);
-  return PlanOut{v.l128, v.l64, v.l32, v.l16, v.counts, narrow};
+  return PlanOut{v.l128, v.l64, v.l32, v.l16, v.counts, narrow, wave_layer(p)};
 }
 
 int launch_prefill_gate_up(hipStream_t s, const PrefillRouted& p) {

@@ -369,20 +369,21 @@ __device__ __forceinline__ int expert_bits(int E) {
 }
 
 // Tiles of one expert with n rows: full 128-row tiles, then the remainder r
-// as one 128-row (r > 64), 64-row (r > 32), 32-row (r > 16) or 16-row tile. The
+// as one 128-row (r > 64), 64-row (r > 32), 32-row (r > 16) or 16-row tile
+// (the general kernels have none: 32-row). The
 // dequantisation cost of a tile does not depend on its row count, the MFMA
 // cost does: small remainders take the cheaper narrow tiles.
 struct TileCounts {
   uint32_t t128, t64, t32, t16;
 };
 // narrow: 16-row tiles only (one launch; batches of few rows per expert).
-__device__ __forceinline__ TileCounts tile_counts(uint32_t n, bool narrow) {
+__device__ __forceinline__ TileCounts tile_counts(uint32_t n, bool narrow, bool t16) {
   if (narrow) return TileCounts{0, 0, 0, (n + 15) / 16};
   const uint32_t r = n % 128;
   TileCounts t{n / 128, 0, 0, 0};
   if (r > 64) t.t128 += 1;
   else if (r > 32) t.t64 = 1;
-  else if (r > 16) t.t32 = 1;
+  else if (r > (t16 ? 16 : 0)) t.t32 = 1;
   else if (r > 0) t.t16 = 1;
   return t;
 }
@@ -439,7 +440,7 @@ __device__ __forceinline__ void dispatch_scan(const uint32_t* count, int E, uint
   uint32_t s128 = 0, s64 = 0, s32 = 0, s16 = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    t4[j] = tile_counts(c4[j], plan.narrow);  // zero for e >= E (c4 is zero there)
+    t4[j] = tile_counts(c4[j], plan.narrow, plan.t16);  // zero for e >= E (c4 is zero there)
     s128 += t4[j].t128;
     s64 += t4[j].t64;
     s32 += t4[j].t32;
