@@ -46,7 +46,7 @@ struct PlanOut {
   uint4* l32;
   uint4* l16;
   uint32_t* counts;  // [4]: lengths of l128, l64, l32, l16
-  bool narrow;       // 16-row tiles only
+  uint32_t narrow;   // experts of at most so many rows: 16-row tiles only
   bool t16;          // 16-row tiles for remainders (else 32-row ones)
 };
 

@@ -1128,12 +1128,12 @@ struct PlanView {
   size_t n128, n64, n32, n16;
 };
 
-PlanView plan_view(uint32_t* plan, size_t A, size_t E, bool narrow) {
+PlanView plan_view(uint32_t* plan, size_t A, size_t E, uint32_t narrow) {
   PlanView v;
   v.n128 = bound128(A, E);
   v.n64 = bound_small(A, E);
   v.n32 = bound_small(A, E);
-  v.n16 = bound16(A, E, narrow);
+  v.n16 = bound16(A, E, narrow != 0);
   v.l128 = reinterpret_cast<uint4*>(plan);
   v.l64 = v.l128 + v.n128;
   v.l32 = v.l64 + v.n64;
@@ -1235,14 +1235,15 @@ int launch_tile128_q(hipStream_t s, int quant, const GemmArgs& a, unsigned grid_
 // -> 145 us, Q4_K 161 -> 195).
 template <int NMAT>
 int launch_tiled(hipStream_t s, int quant, GemmArgs a, const PlanView& v, size_t max_rows,
-                 bool narrow, bool wave) {
+                 uint32_t narrow, bool wave) {
   int st;
+  a.tiles = v.l128;
+  a.n_tiles = v.counts;
+  if (max_rows > std::max<size_t>(64, narrow) &&
+      (st = wave ? launch_tile128_q<NMAT>(s, quant, a, unsigned(v.n128))
+                 : launch_gemm_q<NMAT, 128>(s, quant, a, unsigned(v.n128))))
+    return st;
   if (!narrow) {
-    a.tiles = v.l128;
-    a.n_tiles = v.counts;
-    if (max_rows > 64 && (st = wave ? launch_tile128_q<NMAT>(s, quant, a, unsigned(v.n128))
-                                    : launch_gemm_q<NMAT, 128>(s, quant, a, unsigned(v.n128))))
-      return st;
     a.tiles = v.l64;
     a.n_tiles = v.counts + 1;
     if (max_rows > 32 && (st = wave ? launch_wave_q<NMAT, 4, 3>(s, quant, a, unsigned(v.n64))
@@ -1406,7 +1407,8 @@ bool wave_layer(const PrefillRouted& p) {
   return wave_gemm_takes(p.quant, gate_up_args(p)) && wave_gemm_takes(p.down_quant, down_args(p));
 }
 
-// True when the layer takes 16-row tiles only: one launch per GEMM instead of
+// Rows up to which an expert of the layer takes 16-row tiles only (0: tiles by
+// its remainder): one launch per GEMM instead of
 // one per tile size that an expert could fill, and more workgroups; an expert
 // of more rows reads its weights once per 16 (of which L2 and the Infinity
 // Cache hold the later ones).
@@ -1424,17 +1426,28 @@ bool wave_layer(const PrefillRouted& p) {
 // -> 92; H 6144, I 2048, 16 experts, 1024 (2560), Q2_K 316 -> 236, Q3_K 372 ->
 // 333, 1536 (3584) 255 -> 311, 290 -> 442; H 4096, I 1536, 32 experts, Q3_K,
 // 1024 (2304) even, 1536 (3072) 175 -> 266.
+// The average says nothing of one expert, which may hold all rows of the batch
+// (a caller's routing): above kNarrowMost rows its tiles are of 128 rows, in a
+// launch of their own that such a batch alone needs (0.5 % of an even one).
+// All tokens to 8 of 256 experts of 2048 x 6144, tiles of 16 rows only / 128-row
+// tiles: 128 tokens Q2_K 198 / 216, Q3_K 271 / 245, Q4_K 206 / 211 us, 192 282 /
+// 309, 393 / 379, 295 / 309, 320 453 / 347, 638 / 410, 483 / 355. On the general
+// kernels, which dequantise a matrix once per 16 rows, earlier: 1536 x 4096, 128
+// tokens Q2_K 180 / 124, Q4_K 210 / 224, 320 424 / 202, 493 / 363.
+constexpr uint32_t kNarrowMost = 192, kNarrowMostGeneral = 64;
 constexpr size_t kNarrowRows = 10;
 constexpr size_t kNarrowGroups = 2560;
-bool narrow_layer(const PrefillRouted& p) {
+uint32_t narrow_layer(const PrefillRouted& p) {
   const size_t A = p.T * p.k;
-  return p.h32 != nullptr || A <= kNarrowRows * p.E ||
-         (wave_layer(p) && (p.E + A / 16) * (p.I / 64) <= kNarrowGroups);
+  const bool wave = wave_layer(p);
+  if (p.h32 != nullptr || (wave && (p.E + A / 16) * (p.I / 64) <= kNarrowGroups))
+    return 0xffffffffu;
+  return A > kNarrowRows * p.E ? 0u : wave ? kNarrowMost : kNarrowMostGeneral;
 }
 }  // namespace
 
 PlanOut prefill_plan_out(const PrefillRouted& p) {
-  const bool narrow = narrow_layer(p);
+  const uint32_t narrow = narrow_layer(p);
   const PlanView v = plan_view(p.plan, p.T * p.k, p.E, narrow);
   return PlanOut{v.l128, v.l64, v.l32, v.l16, v.counts, narrow, wave_layer(p)};
 }
@@ -1446,7 +1459,7 @@ int launch_prefill_gate_up(hipStream_t s, const PrefillRouted& p) {
     set_error("MFMA prefill path does not cover this layer");
     return INFERNO_ERR_INVALID;
   }
-  const bool narrow = narrow_layer(p);
+  const uint32_t narrow = narrow_layer(p);
   if (p.h32) return launch_few<2>(s, p.quant, gate_up_args(p), plan_view(p.plan, A, p.E, narrow));
   return launch_tiled<2>(s, p.quant, gate_up_args(p), plan_view(p.plan, A, p.E, narrow),
                          p.max_rows ? p.max_rows : A, narrow, wave_layer(p));
@@ -1455,7 +1468,7 @@ int launch_prefill_gate_up(hipStream_t s, const PrefillRouted& p) {
 int launch_prefill_down(hipStream_t s, const PrefillRouted& p) {
   const size_t A = p.T * p.k;
   if (A == 0) return INFERNO_OK;
-  const bool narrow = narrow_layer(p);
+  const uint32_t narrow = narrow_layer(p);
   if (p.h32) return launch_few<1>(s, p.down_quant, down_args(p), plan_view(p.plan, A, p.E, narrow));
   return launch_tiled<1>(s, p.down_quant, down_args(p), plan_view(p.plan, A, p.E, narrow),
                          p.max_rows ? p.max_rows : A, narrow, wave_layer(p));

@@ -376,12 +376,15 @@ __device__ __forceinline__ int expert_bits(int E) {
 struct TileCounts {
   uint32_t t128, t64, t32, t16;
 };
-// narrow: 16-row tiles only (one launch; batches of few rows per expert).
-__device__ __forceinline__ TileCounts tile_counts(uint32_t n, bool narrow, bool t16) {
-  if (narrow) return TileCounts{0, 0, 0, (n + 15) / 16};
+// narrow: 16-row tiles only for experts of at most so many rows (batches of
+// few rows per expert); the others then take no 64- and 32-row tiles either
+// (where the kernels half fill 16-row tiles, 128-row ones from 33 rows on).
+__device__ __forceinline__ TileCounts tile_counts(uint32_t n, uint32_t narrow, bool t16) {
+  if (n <= narrow) return TileCounts{0, 0, 0, (n + 15) / 16};
   const uint32_t r = n % 128;
   TileCounts t{n / 128, 0, 0, 0};
-  if (r > 64) t.t128 += 1;
+  if (r > 64 || (narrow && !t16 && r > 32)) t.t128 += 1;
+  else if (narrow) t.t16 = (r + 15) / 16;
   else if (r > 32) t.t64 = 1;
   else if (r > (t16 ? 16 : 0)) t.t32 = 1;
   else if (r > 0) t.t16 = 1;

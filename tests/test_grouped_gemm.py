@@ -275,3 +275,15 @@ def test_dense_expert_tiles(quant, down, T, H, Is):
     a, b = (x.double() @ ops.dequantize(quant, sh[i]).view(Is, H).double().T for i in (0, 1))
     ref = (a * torch.sigmoid(a) * b) @ ops.dequantize(down, sh[2]).view(H, Is).double().T
     assert float((out[1] - out[0] - ref).norm() / ref.norm()) < BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,down", PAIRS)
+@pytest.mark.parametrize("shift", [0, 2])
+def test_few_experts_take_all_rows(quant, down, shift):
+    # at most ten rows per expert on average, but two experts hold nearly all:
+    # 128-row tiles with remainders of 1 to 128 rows beside 16-row ones (64
+    # experts of 3072 make more workgroups than the rule of small layers takes)
+    rows = [0] * 64
+    rows[3], rows[17], rows[40], rows[41], rows[63] = 321, 192, 65, 33, 1
+    assert _run(quant, down, 512, 3072, tuple(rows), bf16=True, shift=shift) < BOUND
