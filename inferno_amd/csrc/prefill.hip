@@ -980,10 +980,9 @@ bool gemm2_enabled() {
   return !switch_off("INFERNO_PREFILL_GEMM2");
 }
 
-// Token tiles of whole K units in the 32-token staged GEMMs
-// (INFERNO_PREFILL_XU=0: per 64-deep step).
-bool unit_tokens() { return !switch_off("INFERNO_PREFILL_XU"); }
-
+// The general GEMMs: routed and K-format dense experts whose weights the LDS
+// DMA cannot take, the Q6_K down over 128-row tiles, Q8_0 dense experts. One
+// instance per format, matrix count and tile (and INFERNO_PREFILL_GEMM2=0).
 template <int Q, int NMAT, int TM>
 int launch_gemm(hipStream_t s, const GemmArgs& a, unsigned grid_y) {
   if (grid_y == 0) return INFERNO_OK;
@@ -995,9 +994,8 @@ int launch_gemm(hipStream_t s, const GemmArgs& a, unsigned grid_y) {
   // wavefronts, four workgroups per CU): 468 -> 438 us; c5 layer 5.28 ->
   // 5.22 ms (three A/B pairs); the 64-token down with one LDS weight buffer
   // at four waves per SIMD: 300 -> 221 us, layer 4.93 -> 4.84 ms.
-  // INFERNO_PREFILL_Q2_SMALL_WG=0: the kernels below.
   if constexpr (Q == INFERNO_Q2_K && (TM == 128 || TM == 64) && (NMAT == 1 || TM == 64)) {
-    if (a.N % 128 == 0 && gemm2_enabled() && !switch_off("INFERNO_PREFILL_Q2_SMALL_WG")) {
+    if (a.N % 128 == 0 && gemm2_enabled()) {
       if constexpr (NMAT == 1 && TM == 128) {
         const dim3 g2(unsigned(a.N / 128), grid_y);
         gemm2_kernel<Q, 1, TM, 1, 4, 1, 3, 1, 0><<<g2, 256, gemm2_lds_bytes<Q, 1, TM, 4, 1>(), s>>>(a);
@@ -1018,13 +1016,12 @@ int launch_gemm(hipStream_t s, const GemmArgs& a, unsigned grid_y) {
   // loads). Q3_K prefetches two steps ahead.
   constexpr bool kStaged =
       ((Q == INFERNO_Q2_K || Q == INFERNO_Q3_K) &&
-       (TM <= 64 || (NMAT == 1 && Q == INFERNO_Q3_K) || (NMAT == 2 && Q == INFERNO_Q2_K))) ||
+       (TM == 32 || (NMAT == 2 && Q == INFERNO_Q2_K && TM == 128) ||
+        (Q == INFERNO_Q3_K && (TM == 64 || NMAT == 1)))) ||
       (Q == INFERNO_Q8_0 && (TM == 32 || TM == 128)) ||
       (Q == INFERNO_Q4_K && TM == 32) || (Q == INFERNO_Q6_K && NMAT == 1 && TM == 32);
   if constexpr (kStaged) {
-    // INFERNO_PREFILL_Q4_STAGED=0: Q4_K and Q6_K on the fragment-load kernel
-    if (a.N % 128 == 0 && gemm2_enabled() &&
-        ((Q != INFERNO_Q4_K && Q != INFERNO_Q6_K) || !switch_off("INFERNO_PREFILL_Q4_STAGED"))) {
+    if (a.N % 128 == 0 && gemm2_enabled()) {
       const dim3 grid(unsigned(a.N / 128), grid_y);
       if constexpr (Q == INFERNO_Q8_0 && TM == 128) {
         // Q8_0 (272-byte K units): one weight buffer; gate/up with one
@@ -1044,16 +1041,14 @@ int launch_gemm(hipStream_t s, const GemmArgs& a, unsigned grid_y) {
             <<<grid, 256, gemm2_lds_bytes<Q, 1, TM, 4, 1>(), s>>>(a);
       } else if constexpr (NMAT == 2 && TM == 32) {
         // gate/up over few tokens: one matrix per wavefront (eight), one
-        // weight buffer, four waves per SIMD; token tiles per K unit
-        // (INFERNO_PREFILL_XU=0: per 64-deep step; Q8_0 keeps them per step,
-        // its unit tiles would spill). Fewer than two workgroups per CU of
+        // weight buffer, four waves per SIMD; token tiles per K unit (Q8_0
+        // keeps them per step, its unit tiles would spill). Fewer than two workgroups per CU of
         // 128-row tiles (few experts, narrow I: c1, the XS layer): 64-row
         // tiles on four wavefronts, twice the workgroups, so that more of
         // the weights are in flight per CU
         // (not Q3_K: its 64-row instance spills 18 registers)
         if constexpr (Q == INFERNO_Q2_K || Q == INFERNO_Q4_K) {
-          if (unit_tokens() && size_t(a.N / 128) * grid_y < 2 * kGemmCUs &&
-              !switch_off("INFERNO_PREFILL_NARROW32")) {
+          if (size_t(a.N / 128) * grid_y < 2 * kGemmCUs) {
             const dim3 g2(unsigned(a.N / 64), grid_y);
             gemm2_kernel<Q, 2, TM, 1, 2, 1, 4, 1, 1, 4>
                 <<<g2, 256, gemm2_lds_bytes<Q, 2, TM, 2, 1, 4>(), s>>>(a);
@@ -1061,35 +1056,18 @@ int launch_gemm(hipStream_t s, const GemmArgs& a, unsigned grid_y) {
             return INFERNO_OK;
           }
         }
-        if (Q != INFERNO_Q8_0 && unit_tokens())
-          gemm2_kernel<Q, 2, TM, 1, 4, 1, 4, 1, 1, Q != INFERNO_Q8_0 ? 4 : 0>
-              <<<grid, 512, gemm2_lds_bytes<Q, 2, TM, 4, 1, Q != INFERNO_Q8_0 ? 4 : 0>(), s>>>(a);
-        else
-          gemm2_kernel<Q, 2, TM, 1, 4, 1, 4, 1, 1>
-              <<<grid, 512, gemm2_lds_bytes<Q, 2, TM, 4, 1>(), s>>>(a);
+        constexpr int XU = Q != INFERNO_Q8_0 ? 4 : 0;
+        gemm2_kernel<Q, 2, TM, 1, 4, 1, 4, 1, 1, XU>
+            <<<grid, 512, gemm2_lds_bytes<Q, 2, TM, 4, 1, XU>(), s>>>(a);
       } else if constexpr (NMAT == 2 && TM == 128) {
-        // Q2_K gate/up over 128 tokens: one matrix per wavefront (64
-        // accumulators each), compiled for three waves per SIMD (lab, dense
-        // tiles: 1.81 vs 2.13 ms for the fragment-load kernel; c5 layer:
-        // 5.21 vs 5.29 ms)
-        // INFERNO_PREFILL_XU2=1: token tiles of two steps, one barrier per
-        // two steps, compiled for two waves per SIMD (one 8-wave workgroup
-        // per CU either way)
-        // Default: 64 rows per matrix on four wavefronts (one matrix each) with
-        // one LDS weight buffer, three workgroups per CU, so that three waves
-        // share each SIMD (the 128-row eight-wavefront tile fits one
-        // workgroup per CU: two waves per SIMD): c5 gate/up 1.98 -> 1.85 ms.
-        // INFERNO_PREFILL_G128_WIDE=1: the 128-row tile.
-        if (!switch_on("INFERNO_PREFILL_G128_WIDE") && !switch_on("INFERNO_PREFILL_XU2")) {
-          const dim3 g2(unsigned(a.N / 64), grid_y);
-          gemm2_kernel<Q, 2, TM, 1, 2, 1, 3, 1, 1>
-              <<<g2, 256, gemm2_lds_bytes<Q, 2, TM, 2, 1>(), s>>>(a);
-        } else if (switch_on("INFERNO_PREFILL_XU2"))
-          gemm2_kernel<Q, 2, TM, 1, 4, 1, 2, 0, 1, 2>
-              <<<grid, 512, gemm2_lds_bytes<Q, 2, TM, 4, 0, 2>(), s>>>(a);
-        else
-          gemm2_kernel<Q, 2, TM, 1, 4, 1, 3, 0, 1>
-              <<<grid, 512, gemm2_lds_bytes<Q, 2, TM, 4, 0>(), s>>>(a);
+        // Q2_K gate/up over 128 tokens: 64 rows per matrix on four wavefronts
+        // (one matrix each) with one LDS weight buffer, three workgroups per
+        // CU, so that three waves share each SIMD (a 128-row eight-wavefront
+        // tile fits one workgroup per CU: two waves per SIMD): c5 gate/up 1.98
+        // -> 1.85 ms, layer 5.21 vs 5.29 ms for the fragment-load kernel
+        const dim3 g2(unsigned(a.N / 64), grid_y);
+        gemm2_kernel<Q, 2, TM, 1, 2, 1, 3, 1, 1>
+            <<<g2, 256, gemm2_lds_bytes<Q, 2, TM, 2, 1>(), s>>>(a);
       } else {
         constexpr int PF = Q == INFERNO_Q3_K ? 2 : 1;
         gemm2_kernel<Q, NMAT, TM, PF, 4, 1, 2><<<grid, 256, gemm2_lds_bytes<Q, NMAT, TM, 4>(), s>>>(a);

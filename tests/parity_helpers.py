@@ -27,6 +27,30 @@ def compact_experts(lt, cfg, experts):
     return to_np(g).reshape(-1), to_np(u).reshape(-1), to_np(d).reshape(-1)
 
 
+def moved(t, shift):
+    """The same bytes `shift` past an aligned address."""
+    buf = torch.empty(t.numel() + 16, dtype=torch.uint8, device=t.device)
+    buf[shift:shift + t.numel()] = t
+    return buf[shift:shift + t.numel()]
+
+
+def off_alignment(cfg, lt, max_tokens, shift=2):
+    """Moves a layer's routed matrices `shift` bytes past an aligned address,
+    where the LDS DMA cannot take them, and rebuilds its MoELayer on them."""
+    for name in ("gate", "up", "down"):
+        setattr(lt, name, moved(getattr(lt, name), shift))
+    sg, su, sd = lt.shared or (None, None, None)
+    lt.layer = ops.MoELayer(
+        hidden=cfg.hidden, experts=cfg.experts, intermediate=cfg.intermediate, top_k=cfg.top_k,
+        quant=lt.quant, down_quant=lt.down_quant or lt.quant, score_fn=cfg.score_fn,
+        norm_topk_prob=cfg.norm, routed_scaling_factor=cfg.scale, router=lt.router,
+        router_bias=lt.bias, gate=lt.gate, up=lt.up, down=lt.down,
+        shared_intermediate=cfg.shared_intermediate if lt.shared else 0, shared_gate=sg,
+        shared_up=su, shared_down=sd, shared_quant=lt.shared_quant,
+        shared_down_quant=lt.shared_down_quant, max_tokens=max_tokens)
+    return lt
+
+
 def selection_values(cfg, logits, bias):
     l64 = logits.astype(np.float32)
     if cfg.score_fn == 0:

@@ -329,13 +329,16 @@ def test_rms_norm(cuda):
     assert np.allclose(got, ref, rtol=2e-6, atol=1e-6)
 
 
-def _layer_parity(cuda, key, T, tokens=None, variants=1, tol=None):
+def _layer_parity(cuda, key, T, tokens=None, variants=1, tol=None, shift=0):
     """Layer output against the oracle on `variants` seeded inputs of T tokens
     (rows `tokens` of each; all rows by default). The MoE part's relative L2
     error is taken over all checked rows together and must stay below `tol`
-    (default); returns it."""
+    (default); returns it. shift: the routed matrices
+    lie so many bytes past an aligned address."""
     cfg = cf.CONFIGS[key] if isinstance(key, str) else key
     lt = cf.build_layer(cfg, 0, cuda, max_tokens=T)
+    if shift:
+        lt = ph.off_alignment(cfg, lt, T, shift)
     tokens = np.arange(T) if tokens is None else np.asarray(tokens)
     got_all, ref_all, flips = [], [], 0
     for v in range(variants):
@@ -428,10 +431,17 @@ def test_layer_prefill_shared_ragged_tiles(cuda, T):
 
 
 @pytest.mark.parametrize("key,T", [("c2", 4), ("c2", 8), ("c4", 6)])
-def test_layer_decode_several_tokens_shared(cuda, key, T):
-    # below the grouped GEMM's 66 assignments with a Q8_0 shared expert: the
-    # several-token decode launches (select, packed-f16 tiles), full size
+@pytest.mark.parametrize("side,kernel", [("0", "tiles: gate_up_kernel"),
+                                         (None, "grouped, few tokens: gate/up GEMM")])
+def test_layer_decode_several_tokens_shared(cuda, switches, key, T, side, kernel):
+    # below the grouped GEMM's 66 assignments with a Q8_0 shared expert, full
+    # size: the several-token decode launches (select, packed-f16 tiles), and
+    # by the rule the grouped GEMMs over scaled rows
+    if side:
+        switches(INFERNO_DECODE_GROUPED=side)
     _layer_parity(cuda, key, T)
+    labels, _ = _labels_of_one_step(cf.CONFIGS[key], cuda, T)
+    assert labels[ops.TIMER_GATE_UP].startswith(kernel), labels
 
 
 @pytest.mark.parametrize("T", [1, 16])
@@ -665,18 +675,17 @@ def c5_check_tokens(ids, T, k, E):
     return np.array(sorted(rows)), load, sorted(classes)
 
 
-@pytest.mark.parametrize("variant", ["default", "wide"])
-def test_layer_c5_glm_q2k_prefill_zipf(cuda, switches, variant):
+@pytest.mark.parametrize("variant", ["default", "general"])
+def test_layer_c5_glm_q2k_prefill_zipf(cuda, variant):
     # full-size skewed prefill: router bias fitted so the load follows
     # Zipf(1.1) over 216 experts (hottest capped at one slot per token,
-    # 12.5%), 40 experts without a token. "wide": the Q2_K GEMMs on their
-    # larger-workgroup kernels (INFERNO_PREFILL_Q2_SMALL_WG=0,
-    # INFERNO_PREFILL_G128_WIDE=1), against the same oracle bound
-    if variant == "wide":
-        switches(INFERNO_PREFILL_Q2_SMALL_WG="0", INFERNO_PREFILL_G128_WIDE="1")
+    # 12.5%), 40 experts without a token. "general": matrices that the LDS
+    # DMA cannot take, on the general GEMMs, against the same oracle bound
     cfg = cf.CONFIGS["c5"]
     T, k, E = 4096, cfg.top_k, cfg.experts
     lt = cf.build_layer(cfg, 0, cuda, max_tokens=T)
+    if variant == "general":
+        lt = ph.off_alignment(cfg, lt, T)
     x = cf.make_input(cfg, T, device=cuda)
     logits = ops.router_logits(x, lt.router)
     lt.bias.copy_(torch.from_numpy(cf.zipf_bias(cfg, ph.to_np(logits))).to(cuda))
@@ -850,11 +859,11 @@ def switches(monkeypatch):
 
 
 def test_layer_prefill_fragment_kernel_variant(cuda, switches):
-    """The prefill GEMMs all on the fragment-load kernel and the fp32 router
-    logits (INFERNO_PREFILL_GEMM2=0, INFERNO_ROUTER_BF16X3=0): c3, every
-    token, against the oracle."""
+    """The general GEMMs all on the fragment-load kernel and the fp32 router
+    logits (INFERNO_PREFILL_GEMM2=0, INFERNO_ROUTER_BF16X3=0): c3 with matrices
+    that the LDS DMA cannot take, every token, against the oracle."""
     switches(INFERNO_PREFILL_GEMM2="0", INFERNO_ROUTER_BF16X3="0")
-    _layer_parity(cuda, "c3", 512)
+    _layer_parity(cuda, "c3", 512, shift=2)
 
 
 @pytest.mark.parametrize("key", ["c2", "c4"])
