@@ -14,7 +14,7 @@ def _weights(quant, seed, rows, cols):
     return ops.synth_quantized(quant, seed, 0.02, rows, cols, torch.device("cuda:0"))
 
 
-def _layer(quant, shared, T, router_std=0.02, E=E, k=TOP_K):
+def _layer(quant, shared, T, router_std=0.02, E=E, k=TOP_K, tensors=None):
     g = torch.Generator(device="cuda").manual_seed(2)
     kw = {}
     if shared:
@@ -26,7 +26,7 @@ def _layer(quant, shared, T, router_std=0.02, E=E, k=TOP_K):
         hidden=H, experts=E, intermediate=I, top_k=k, quant=quant, down_quant=quant,
         score_fn=SCORE_SOFTMAX, norm_topk_prob=True, routed_scaling_factor=1.0,
         router=torch.randn(E, H, generator=g, device="cuda") * router_std, router_bias=None,
-        shared_intermediate=IS if shared else 0, max_tokens=T, **mats, **kw)
+        shared_intermediate=IS if shared else 0, max_tokens=T, **(tensors or dict(mats, **kw)))
     return layer, mats, kw
 
 
@@ -143,3 +143,25 @@ def test_rule(quant, T, hands_over, shared, monkeypatch):
     by_rule, decode, grouped = _sides(monkeypatch, layer, x)
     assert not torch.equal(decode, grouped)
     assert torch.equal(by_rule, grouped if hands_over else decode)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant", [Q2_K, Q3_K, Q4_K])
+@pytest.mark.parametrize("moved,shift", [("gate", 2), ("up", 4), ("down", 8), ("shared_gate", 2),
+                                         ("shared_down", 8)])
+def test_matrices_off_the_dma(quant, moved, shift, monkeypatch):
+    # a matrix that the LDS DMA cannot take (routed: whole words, Q4_K 16 bytes;
+    # shared: 16 bytes) keeps the layer on the decode launches, also when asked
+    # for the GEMMs; one that it can take does not
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(6, H, generator=g, device="cuda").bfloat16()
+    _, mats, sh = _layer(quant, True, 6)
+    t = dict(mats, **sh)
+    buf = torch.empty(t[moved].numel() + 16, dtype=torch.uint8, device="cuda")
+    buf[shift:shift + t[moved].numel()] = t[moved]
+    t[moved] = buf[shift:shift + t[moved].numel()]
+    layer, _, _ = _layer(quant, True, 6, tensors=t)
+    by_rule, decode, forced = _sides(monkeypatch, layer, x)
+    taken = shift % 4 == 0 and quant != Q4_K and not moved.startswith("shared")
+    assert torch.equal(forced, decode) == (not taken)
+    assert torch.equal(by_rule, forced if quant == Q3_K or not taken else decode)

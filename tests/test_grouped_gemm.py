@@ -146,9 +146,12 @@ def test_sixteen_row_tiles_only(quant, down):
 @pytest.mark.gpu
 @pytest.mark.parametrize("quant,down", PAIRS)
 @pytest.mark.parametrize("shift", [2, 4])
-def test_weights_at_any_address(quant, down, shift):
-    # 2 bytes past a word (and 4 past 16 bytes for Q4_K): not the DMA's rows
-    assert _run(quant, down, 512, 256, (18, 30, 4, 0), bf16=True, shift=shift) < BOUND
+@pytest.mark.parametrize("H,I", [(512, 256), (768, 1280), (256, 768)])
+def test_weights_at_any_address(quant, down, shift, H, I):
+    # 2 bytes past a word (and 4 past 16 bytes for Q4_K): not the DMA's rows;
+    # even and odd super-block counts, tiles of 32, 64 and 128 rows
+    assert _run(quant, down, H, I, (18, 30, 4, 0), bf16=True, shift=shift) < BOUND
+    assert _run(quant, down, H, I, (40, 150, 17, 77), bf16=True, shift=shift) < BOUND
 
 
 @pytest.mark.gpu
@@ -217,9 +220,10 @@ def test_dense_q8_rows_beside_a_large_value(T, bf16):
 @pytest.mark.parametrize("shared", [0, 1024])
 @pytest.mark.parametrize("quant", [Q2_K, Q3_K, Q4_K])
 def test_layer_decode_and_grouped_agree(quant, shared, T, monkeypatch):
-    # both sides of the rule that hands a few tokens to the grouped GEMMs: the
-    # same layer on the fused decode launches (a threshold no batch reaches)
-    # and by the rule, outputs within the rounding of h to f16 (2^-12 each)
+    # the three paths of a few tokens: the fused decode launches (a threshold no
+    # batch reaches; the rule keeps these there but for Q3_K and Q4_K of six
+    # tokens), the grouped GEMMs over scaled rows and over plain ones (a
+    # threshold of 1); outputs within the rounding of h to f16 (2^-12 each)
     from inferno_amd import Q8_0, SCORE_SOFTMAX
     dev = torch.device("cuda:0")
     H, E, I, k = 3072, 32, 1024, 6
@@ -236,11 +240,16 @@ def test_layer_decode_and_grouped_agree(quant, shared, T, monkeypatch):
         shared_down=sh[2], max_tokens=T)
     x = torch.randn(T, H, generator=g, device=dev).bfloat16()
     by_rule = layer.forward(x)
+    monkeypatch.setenv("INFERNO_DECODE_GROUPED", "1")
+    scaled = layer.forward(x)
+    monkeypatch.delenv("INFERNO_DECODE_GROUPED")
     monkeypatch.setenv("INFERNO_PREFILL_MIN_ASSIGNMENTS", "100000")
     decode = layer.forward(x)
     monkeypatch.setenv("INFERNO_PREFILL_MIN_ASSIGNMENTS", "1")
     grouped = layer.forward(x)
-    assert float((by_rule - decode).norm() / decode.norm()) < 2e-3
+    assert torch.equal(by_rule, scaled if T == 6 and quant != Q2_K else decode)
+    assert not torch.equal(scaled, decode) and not torch.equal(grouped, decode)
+    assert float((scaled - decode).norm() / decode.norm()) < 2e-3
     assert float((grouped - decode).norm() / decode.norm()) < 2e-3
 
 
