@@ -205,7 +205,7 @@ __device__ __forceinline__ void stage_run_lanes_mfma(float v, uint32_t* row, int
   if (m > 0.f && m < 3.0e38f) {
     int e;
     frexpf(m, &e);
-    s = ldexpf(1.0f, 15 - e);
+    s = ldexpf(1.0f, min(15 - e, 126));  // (finite below 2^-111 too)
   }
   const int p = ((run & 15) >> 1) & 3;  // bit plane of this run's group
   const _Float16 hv = (_Float16)(v * (s * ldexpf(1.0f, -2 * p)));

@@ -359,7 +359,7 @@ __device__ __forceinline__ void stage_run16(float v, uint32_t* row, int K, int r
   if (m > 0.f && m < 3.0e38f) {
     int e;
     frexpf(m, &e);
-    s = ldexpf(1.0f, 15 - e);
+    s = ldexpf(1.0f, min(15 - e, 126));  // (finite below 2^-111 too)
   }
   const float vs = v * (s * ldexpf(1.0f, -shift));
   const _Float16 hv = (_Float16)vs;

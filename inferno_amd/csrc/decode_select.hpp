@@ -118,7 +118,7 @@ struct SharedHQuad {
     if (m > 0.f && m < 3.0e38f) {
       int e;
       frexpf(m, &e);
-      scale = ldexpf(1.0f, 15 - e);
+      scale = ldexpf(1.0f, min(15 - e, 126));  // (finite below 2^-111 too)
     }
     auto pack = [](float a, float b) {
       const _Float16 ah = (_Float16)a, bh = (_Float16)b;

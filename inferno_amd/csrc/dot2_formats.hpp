@@ -102,7 +102,7 @@ __device__ __forceinline__ void stage_run(const float v[16], uint32_t* row, int 
   if (m > 0.f && m < 3.0e38f) {
     int e;
     frexpf(m, &e);  // m = f * 2^e, f in [0.5, 1)
-    scale = ldexpf(1.0f, 15 - e);
+    scale = ldexpf(1.0f, min(15 - e, 126));  // (finite below 2^-111 too)
   }
   uint32_t* hi = row + run * 8;
 #pragma unroll
@@ -457,7 +457,7 @@ __device__ __forceinline__ void stage_run_lanes(float v, uint32_t* row, int K, i
   if (m > 0.f && m < 3.0e38f) {
     int e;
     frexpf(m, &e);
-    scale = ldexpf(1.0f, 15 - e);
+    scale = ldexpf(1.0f, min(15 - e, 126));  // (finite below 2^-111 too)
   }
   const float a = v * scale;
   const _Float16 ah = (_Float16)a;

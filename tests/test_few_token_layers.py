@@ -165,3 +165,23 @@ def test_matrices_off_the_dma(quant, moved, shift, monkeypatch):
     taken = shift % 4 == 0 and quant != Q4_K and not moved.startswith("shared")
     assert torch.equal(forced, decode) == (not taken)
     assert torch.equal(by_rule, forced if quant == Q3_K or not taken else decode)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 2, 5])
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("quant", [Q2_K, Q3_K, Q4_K])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_vanishing_routing_weights(quant, shared, T, bf16):
+    # router logits of a standard deviation of 60: softmax weights down to
+    # 1e-38 and below, whose runs of h are subnormal or nearly so
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(T, H, generator=g, device="cuda")
+    x = x.bfloat16() if bf16 else x
+    layer, mats, sh = _layer(quant, shared, T, router_std=60 / H ** 0.5)
+    ids = torch.empty(T * TOP_K, dtype=torch.int32, device="cuda")
+    w = torch.empty(T * TOP_K, device="cuda")
+    y = layer.forward(x, None, ids=ids, weights=w)
+    assert 0 < float(w[w > 0].min()) < 1e-33  # such weights are there
+    ref = _exact(quant, mats, sh, x, ids.view(T, TOP_K), w.view(T, TOP_K))
+    assert float(((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).max()) < DECODE
