@@ -128,6 +128,13 @@ bool use_mfma(int quant, int down_quant, size_t T, size_t k, size_t E, size_t H,
          prefill_routed_supported(quant, down_quant, H, I, E);
 }
 
+constexpr const char* kGroupedGateUp =
+    "prefill: grouped gate/up GEMMs (wave_gemm_kernel / tile128_gemm_kernel; gemm_kernel / "
+    "gemm2_kernel where the LDS DMA cannot take the weights)";
+constexpr const char* kGroupedDown =
+    "prefill: grouped down GEMMs (wave_gemm_kernel / tile128_gemm_kernel; gemm_kernel / "
+    "gemm2_kernel where the LDS DMA cannot take the weights and for Q6_K 128-row tiles)";
+
 // `x16`: x already converted to f16 (MFMA path), or null. `distinct_ids`:
 // every token's k ids are distinct (the layer's own top-k), so one expert
 // takes at most T rows (caller ids may repeat an expert within a token).
@@ -146,10 +153,10 @@ int run_routed(hipStream_t s, int quant, int down_quant, const void* gate, const
     const PlanOut plan = prefill_plan_out(p);
     if ((st = launch_dispatch(s, ids, T, k, E, m.offsets, m.sorted, m.active, &plan))) return st;
     if (conv && (st = launch_to_f16(s, x, x_dtype, T, H, conv))) return st;
-    if ((st = timed(s, kTimerGateUp, "prefill: grouped gate/up GEMMs (gemm_kernel / gemm2_kernel, MFMA)",
+    if ((st = timed(s, kTimerGateUp, kGroupedGateUp,
                     [&] { return launch_prefill_gate_up(s, p); })))
       return st;
-    return timed(s, kTimerDown, "prefill: grouped down GEMMs (gemm_kernel / gemm2_kernel, MFMA)",
+    return timed(s, kTimerDown, kGroupedDown,
                  [&] { return launch_prefill_down(s, p); });
   }
   if ((st = launch_dispatch(s, ids, T, k, E, m.offsets, m.sorted, m.active, nullptr))) return st;
@@ -707,13 +714,13 @@ int layer_few(hipStream_t s, const inferno_moe_layer* L, const void* x, int x_dt
   if ((st = launch_dispatch(s, ids, T, k, E, w.moe.offsets, w.moe.sorted, w.moe.active, &plan)))
     return st;
   if ((st = launch_scaled_rows(s, x_dtype, {x, x16, T, H}, {}))) return st;
-  if ((st = timed(s, kTimerGateUp, "grouped, few tokens: gate/up GEMM (wave_gemm_kernel, scaled rows)",
+  if ((st = timed(s, kTimerGateUp, "prefill: few tokens, gate/up GEMM (wave_gemm_kernel, scaled rows)",
                   [&] { return launch_prefill_gate_up(s, p); })))
     return st;
   if (Is && (st = launch_dense_q8(s, g))) return st;
   if ((st = launch_scaled_rows(s, INFERNO_F32, {w.moe.h, h16, A, I}, {w.hs, hs16, Is ? T : 0, Is})))
     return st;
-  if ((st = timed(s, kTimerDown, "grouped, few tokens: down GEMM (wave_gemm_kernel, scaled rows)",
+  if ((st = timed(s, kTimerDown, "prefill: few tokens, down GEMM (wave_gemm_kernel, scaled rows)",
                   [&] { return launch_prefill_down(s, p); })))
     return st;
   if (Is && (st = launch_dense_q8(s, d))) return st;
@@ -754,10 +761,6 @@ int layer_forward(void* stream, const inferno_moe_layer* L, const void* x, int x
     if ((st = check_len("shared down", L->shared_down_bytes, 1, matrix_bytes(sdq, H, Is))))
       return st;
   }
-  // the fused decode launches and the dense MFMA shared GEMMs take a Q8_0
-  // shared expert (the GLM and Laguna S layers); other formats (Laguna XS:
-  // Q4_K gate/up, Q4_K or Q6_K down) run the shared expert on the GEMV kernels
-  const bool shared_q8 = Is == 0 || (sq == INFERNO_Q8_0 && sdq == INFERNO_Q8_0);
   size_t need = layer_workspace_bytes(L, T, lib);
   if (workspace_bytes < need) {
     set_error("workspace too small: need " + std::to_string(need) + " bytes");

@@ -32,8 +32,9 @@
 namespace inferno {
 namespace {
 
-// Tokens from which the shared expert takes the library GEMMs (below it the
-// grouped kernels' dense path): every prefill batch. Measured against the
+// Tokens from which the shared expert can take the library GEMMs: any that
+// dense_q8_kernel leaves (launch_prefill_dense: more than 128 tokens, or Q8_0
+// weights off 16 bytes, which would else run on the general GEMMs). Measured against the
 // dense path: c2 T = 12 0.462 -> 0.401 ms, c2 T = 16 0.511 -> 0.445, c4
 // T = 12 1.389 -> 1.236, T = 32 1.830 -> 1.650, T = 64 1.888 -> 1.733 (the
 // dense path's 32-row tiles gave a 1536-row shared expert 48 workgroups).

@@ -370,6 +370,7 @@ struct W<INFERNO_Q6_K> {
     const float dsc = d * float(int8_t((sc[T >> 1] >> (16 * (T & 1))) & 0xffu));
     return dequant8(w0, w1, 0x003f003fu, __builtin_amdgcn_ldexpf(dsc, 24), -32.0f * dsc);
   }
+  // (named in code that kExact leaves out, never called)
   __device__ static half8 offsets(const uint32_t*, int, uint32_t) { return half8{}; }
   __device__ static float dscale(const uint32_t*, uint32_t) { return 1.f; }
   __device__ static float mscale(const uint32_t*) { return 0.f; }

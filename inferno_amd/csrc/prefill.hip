@@ -9,11 +9,16 @@
 // combine), which also run the expert products on f16 operands with fp32
 // accumulation.
 //
-// Work item: 128 weight rows (gate and up rows together for the SwiGLU pass)
-// x TM dispatch rows (TM = 128, or 32 for an expert's small remainder). Each
-// wavefront owns 32 weight rows and all TM tokens, issuing
-// v_mfma_f32_32x32x16_f16 with the weights as the A operand and the tokens
-// as B. Every lane dequantises its own A fragments (8 values of one row per
+// The GEMMs themselves are in grouped_gemm.hpp (tiles of up to 64 dispatch
+// rows) and grouped_gemm128.hpp, which bring every operand to LDS by its DMA.
+// Here are their launchers and rules, the conversions and the combine, and the
+// general GEMMs (gemm_kernel, gemm2_kernel) for what the DMA cannot take: other
+// alignments, Q6_K downs over 128-row tiles, Q8_0 dense experts.
+//
+// The general GEMMs' work item: 128 weight rows (gate and up rows together for
+// the SwiGLU pass) x TM dispatch rows (TM = 32, 64 or 128). Each wavefront owns
+// 32 weight rows and all TM tokens, issuing v_mfma_f32_32x32x16_f16 with the
+// weights as the A operand and the tokens as B. Every lane dequantises its own A fragments (8 values of one row per
 // 16-deep k step) straight from the GGUF bytes: a quant field masked in place
 // out of a 32-bit word, at bits p and 16 + p, is a pair of exact f16
 // subnormals q * 2^(p-24), and one v_fma_mix per value (f16 field, fp32
@@ -21,9 +26,10 @@
 // mask takes bytes 0 and 2 (then 1 and 3) of a word, so within every group of
 // eight k the operands run in the order 0 2 1 3 4 6 5 7; the f16 activations
 // (x16, h16) are stored in that same order, which leaves the sum unchanged.
-// The token tile (TM x 64 f16) is double buffered in LDS. Tiles come from a
-// per-expert list built on the device from the dispatch, so nothing waits on
-// the host.
+// The token tile (TM x 64 f16) is double buffered in LDS.
+//
+// Tiles come from a per-expert list built on the device from the dispatch, so
+// nothing waits on the host.
 #include "prefill.hpp"
 
 #include <algorithm>

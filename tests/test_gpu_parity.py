@@ -432,7 +432,7 @@ def test_layer_prefill_shared_ragged_tiles(cuda, T):
 
 @pytest.mark.parametrize("key,T", [("c2", 4), ("c2", 8), ("c4", 6)])
 @pytest.mark.parametrize("side,kernel", [("0", "tiles: gate_up_kernel"),
-                                         (None, "grouped, few tokens: gate/up GEMM")])
+                                         (None, "prefill: few tokens, gate/up GEMM")])
 def test_layer_decode_several_tokens_shared(cuda, switches, key, T, side, kernel):
     # below the grouped GEMM's 66 assignments with a Q8_0 shared expert, full
     # size: the several-token decode launches (select, packed-f16 tiles), and
