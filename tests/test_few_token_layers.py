@@ -185,3 +185,23 @@ def test_vanishing_routing_weights(quant, shared, T, bf16):
     assert 0 < float(w[w > 0].min()) < 1e-33  # such weights are there
     ref = _exact(quant, mats, sh, x, ids.view(T, TOP_K), w.view(T, TOP_K))
     assert float(((y.double() - ref).norm(dim=1) / ref.norm(dim=1)).max()) < DECODE
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shared", [False, True])
+def test_replayed_graph(shared):
+    # the launches of a captured layer read each replay's tokens
+    g = torch.Generator(device="cuda").manual_seed(3)
+    layer, _, _ = _layer(Q3_K, shared, 6)
+    x = torch.randn(6, H, generator=g, device="cuda").bfloat16()
+    out = torch.empty(6, H, device="cuda")
+    layer.forward(x, out=out)  # the kernels' first launches are not captured
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        layer.forward(x, out=out)
+    for _ in range(3):
+        x.copy_((torch.randn(6, H, generator=g, device="cuda") * 50).bfloat16())
+        graph.replay()
+        got = out.clone()
+        assert torch.equal(got, layer.forward(x))
