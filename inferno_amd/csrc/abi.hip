@@ -561,9 +561,10 @@ LayerScratch carve_layer(Carver& c, const inferno_moe_layer* L, size_t T, bool l
   s.moe = carve_moe(c, T, L->top_k, L->experts, L->hidden, L->intermediate);
   // router logits, or their K-chunk partials for a small batch: read by the
   // top-k, before the down rows are written over them. (So the need is linear
-  // in T: the number of chunks is not, it falls as T grows.)
+  // in T: the number of chunks is not, it falls as T grows. A layer has at most
+  // 256 experts and at least 256 columns, so that one chunk always fits.)
   s.logits_parts = std::max<size_t>(1, L->top_k * L->hidden / std::max<size_t>(1, L->experts));
-  s.logits = L->top_k * L->hidden >= L->experts ? s.moe.y : c.take<float>(T * L->experts);
+  s.logits = s.moe.y;
   s.partials = c.take<float>(size_t(L->hidden / decode_chunk(L->hidden)) * T * L->experts);
   s.ys = c.take<float>(T * L->hidden);
   s.slots = c.take<uint4>(L->experts);

@@ -205,3 +205,31 @@ def test_replayed_graph(shared):
         graph.replay()
         got = out.clone()
         assert torch.equal(got, layer.forward(x))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("T", [1, 5, 33, 130])
+def test_router_logits_in_the_down_rows(T, bf16):
+    # the narrowest down rows for the most experts: as many chunks of logits as
+    # their region holds (one, two), ids and weights as the router alone gives
+    from inferno_amd import SCORE_SIGMOID
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for Hn, k in ((256, 1), (256, 2), (512, 1)):
+        x = torch.randn(T, Hn, generator=g, device="cuda")
+        x = x.bfloat16() if bf16 else x
+        router = torch.randn(256, Hn, generator=g, device="cuda") * 0.05
+        layer = ops.MoELayer(
+            hidden=Hn, experts=256, intermediate=256, top_k=k, quant=Q4_K, down_quant=Q4_K,
+            score_fn=SCORE_SIGMOID, norm_topk_prob=False, routed_scaling_factor=1.0, router=router,
+            router_bias=None, gate=_weights(Q4_K, 0, 256 * 256, Hn), up=_weights(Q4_K, 1, 256 * 256, Hn),
+            down=_weights(Q4_K, 2, 256 * Hn, 256), max_tokens=T)
+        ids = torch.empty(T * k, dtype=torch.int32, device="cuda")
+        w = torch.empty(T * k, device="cuda")
+        layer.forward(x, None, ids=ids, weights=w)
+        score = torch.sigmoid(x.double() @ router.double().T)
+        top = score.topk(k, dim=1)
+        # the chosen experts' own scores, and no better one left out (1e-6: ties)
+        got = score.gather(1, ids.view(T, k).long())
+        assert float((got - w.view(T, k)).abs().max()) < 1e-6
+        assert float((top.values - got.sort(dim=1, descending=True).values).abs().max()) < 1e-6
